@@ -30,7 +30,9 @@ COMMON = [
 
 SOURCES = [
     # (source, extra flags)
-    ("sfe_kernels.hip", ["-x", "hip"]),
+    # (the atomic optimizer would broadcast the work counter's lane-0 add, and
+    # wait for it, where it is issued instead of a quad later)
+    ("sfe_kernels.hip", ["-x", "hip", "-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]),
     ("sfe_vad.hip", ["-x", "hip"]),
     ("sfe_noalloc.hip", ["-x", "hip"]),
     # bit-exact table construction: every f32/f64 op rounded separately

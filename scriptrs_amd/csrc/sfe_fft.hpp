@@ -205,4 +205,99 @@ __host__ __device__ __forceinline__ void split_power(cf A, cf B, float s, float 
   pm = fmaf(xm.y, xm.y, xm.x * xm.x);
 }
 
+// 8-point DCT-II of g[0..5], 0, 0: sum over i of g[i] cos(pi k (2 i + 1) /
+// 16), as x[k] times the scale kDct8[k], which the caller applies in its
+// fmas.
+namespace fftc {
+constexpr float kK1 = 0.98078528040323045f;  // cos(pi/16)
+constexpr float kA3 = 0.84775906502257351f;  // cos(3 pi/16) / cos(pi/16)
+constexpr float kA5 = 0.56645449735052156f;  // cos(5 pi/16) / cos(pi/16)
+constexpr float kA7 = 0.19891236737965801f;  // cos(7 pi/16) / cos(pi/16)
+}  // namespace fftc
+__host__ __device__ __forceinline__ void dct8_6(const float (&g)[6], float (&x)[8]) {
+  using namespace fftc;
+  const float s2 = g[2] + g[5], d2 = g[2] - g[5];
+  const float s3 = g[3] + g[4], d3 = g[3] - g[4];
+  const float a = g[0] + s3, c = g[0] - s3;
+  const float b = g[1] + s2, d = g[1] - s2;
+  x[0] = a + b;
+  x[4] = a - b;
+  x[2] = fmaf(kT1, d, c);
+  x[6] = fmaf(kT1, c, -d);
+  x[1] = fmaf(kA7, d3, fmaf(kA5, d2, fmaf(kA3, g[1], g[0])));
+  x[3] = fmaf(-kA3, g[0], fmaf(kA7, g[1], fmaf(kA5, d3, d2)));
+  x[5] = fmaf(-kA3, d3, fmaf(-kA7, d2, fmaf(-kA5, g[0], g[1])));
+  x[7] = fmaf(-kA7, g[0], fmaf(kA5, g[1], fmaf(-kA3, d2, d3)));
+}
+
+// 32-point DFT of the real, windowed inputs v[i] = w[i] y[i] at positions b
+// = i - 12 (i < 25; the other 7 positions are zero), into Y[k] = sum over b
+// of v e^{-2 pi i k b / 32}: Y[k] at y[k] for 0 < k < 16, and the real Y[0]
+// and Y[16] as y[0] = (Y[0], Y[16]).
+//
+// With the origin at the middle input, the real part takes the sums of the
+// pairs +-b and the imaginary part their differences (the window product
+// rides in both), and each half splits again by the parity of b: cosines or
+// sines of even b are a 16-point transform of the same kind, those of odd b
+// an 8-point DCT-II (dct8_6; sin(pi k m / 16) = +-cos(pi (8 - k) m / 16) for
+// odd m).  153 operations, against 154 of the windowed complex 16-point DFT
+// (dft16_windowed), which transforms half as much.
+__host__ __device__ __forceinline__ void rdft32_windowed(const float (&y)[25], const float (&w)[25], cf (&Y)[16]) {
+  using namespace fftc;
+  float e[13], o[13];
+#pragma unroll
+  for (int b = 1; b <= 12; ++b) {
+    const float m = w[12 - b] * y[12 - b];
+    e[b] = fmaf(w[12 + b], y[12 + b], m);
+    // odd b: the sign (-1)^((b - 1) / 2) of the sine's DCT-II form
+    o[b] = b % 4 == 3 ? fmaf(-w[12 + b], y[12 + b], m) : fmaf(w[12 + b], y[12 + b], -m);
+  }
+  e[0] = w[12] * y[12];
+  // cosines, even b: ev[k] = sum over j of e[2 j] cos(pi k j / 8), k <= 8
+  float ev[9], od[8];
+  {
+    const float u = e[0] + e[8], d = e[0] - e[8], p = e[4] + e[12], q = e[4] - e[12];
+    const float g = e[6] + e[10], t = e[6] - e[10];
+    const float z0 = u + p, z1 = fmaf(kR, q, e[0]), z3 = fmaf(-kR, q, e[0]);
+    const float o0 = e[2] + g, o2 = e[2] - g, o1 = fmaf(kT1, t, e[2]), o3 = fmaf(kT1, e[2], -t);
+    ev[0] = z0 + o0;
+    ev[8] = z0 - o0;
+    ev[1] = fmaf(kC1, o1, z1);
+    ev[7] = fmaf(-kC1, o1, z1);
+    ev[2] = fmaf(kR, o2, d);
+    ev[6] = fmaf(-kR, o2, d);
+    ev[3] = fmaf(kC1, o3, z3);
+    ev[5] = fmaf(-kC1, o3, z3);
+    ev[4] = u - p;
+    const float h[6] = {e[1], e[3], e[5], e[7], e[9], e[11]};
+    dct8_6(h, od);
+  }
+  // sines, even b: se[k] = sum over j of o[2 j] sin(pi k j / 8), 1 <= k <= 7
+  float se[8], so[8];
+  {
+    const float v = o[4] + o[12], s2 = o[4] - o[12], s1 = fmaf(kR, v, o[8]), s3 = fmaf(kR, v, -o[8]);
+    const float m1 = o[6] + o[10], m2 = o[6] - o[10];
+    const float h1 = fmaf(kT1, o[2], m1), h3 = fmaf(-kT1, m1, o[2]), h2 = o[2] + m2;
+    se[1] = fmaf(kC1, h1, s1);
+    se[7] = fmaf(kC1, h1, -s1);
+    se[2] = fmaf(kR, h2, s2);
+    se[6] = fmaf(kR, h2, -s2);
+    se[3] = fmaf(kC1, h3, s3);
+    se[5] = fmaf(kC1, h3, -s3);
+    se[4] = o[2] - m2;
+    const float h[6] = {o[1], o[3], o[5], o[7], o[9], o[11]};
+    dct8_6(h, so);  // so[8 - k]: the sum over odd b at k
+  }
+  constexpr float sc[8] = {1.0f, kK1, kC1, -kK1, kR, -kK1, kC1, -kK1};
+  Y[0] = {ev[0] + od[0], ev[0] - od[0]};
+  Y[8] = {ev[8], -so[0]};
+#pragma unroll
+  for (int k = 1; k < 8; ++k) {
+    Y[k].x = fmaf(sc[k], od[k], ev[k]);
+    Y[16 - k].x = fmaf(-sc[k], od[k], ev[k]);
+    Y[k].y = fmaf(-sc[8 - k], so[8 - k], -se[k]);
+    Y[16 - k].y = fmaf(-sc[8 - k], so[8 - k], se[k]);
+  }
+}
+
 }  // namespace sfe

@@ -18,40 +18,31 @@ constexpr int kMel = 128;
 constexpr int kBins = kNfft / 2 + 1;  // 257
 constexpr int kPad = kNfft / 2;       // 256 zeros each side (src/frontend.rs:124-125)
 
-// Mel contraction schedule for v_mfma_f32_4x4x1_16b_f32.  One wave
-// contracts the power spectra of its own 4 frames: an MFMA is 16 blocks of
-// [4 filters x 1 bin] . [1 bin x 4 frames].  Chain 0 holds the blocks of
-// filters 0..63 (block j: filters 4j..4j+3), chain 1 those of filters
-// 64..127.  Block j of chain c runs kChainSteps[schedule][c] consecutive
-// bins from its own first bin (a multiple of 4, from the device table), so
-// the dense 128x257 product is never formed.  Schedule 0 fits the Slaney
-// filterbank at 16, 22.05 and 24 kHz (at 16 kHz the widest block of chain 0
-// spans 7 bins, of chain 1 32); schedule 1, with 50% more steps, fits the
-// other sample rates from 3.5 to 107 kHz (at 8 kHz chain 0 needs 10 bins,
-// at 48 kHz chain 1 needs 41).  The tables take the first that fits.
-constexpr int kChains = 2;
+// Mel contraction schedule.  One wave contracts the power spectra of its own
+// 4 frames: lane L sums filters L and 64 + L (slots 0 and 1) of all 4, slot i
+// over kMelSteps[schedule][i] consecutive bins from the filter's own first
+// bin (from the device table), so the dense 128x257 product is never formed.
+// Schedule 0 fits the Slaney filterbank at 16, 22.05 and 24 kHz (504 nonzero
+// weights); schedule 1 the other sample rates taken (build_dev_tables).
 constexpr int kSchedules = 2;
-constexpr int kChainSteps[kSchedules][kChains] = {{8, 32}, {12, 48}};
-constexpr int mel_vec(int schedule) { return (kChainSteps[schedule][0] + kChainSteps[schedule][1]) / 4; }
-// Power-spectrum bins each schedule's FFT stage writes per frame: the 257
-// bins, and for schedule 1 three zeros after them, so that a block whose
-// filters reach bin 256 can start at a multiple of 4 (the float4 operand
-// loads) and still run its 48 steps inside the written bins.
-constexpr int kBinsWritten[kSchedules] = {kBins, kBins + 3};
-constexpr int kMelVecMax = mel_vec(1);  // float4 A operands per lane, either schedule
-static_assert(kChainSteps[0][0] % 4 == 0 && kChainSteps[0][1] % 4 == 0 && kChainSteps[1][0] % 4 == 0 &&
-                  kChainSteps[1][1] % 4 == 0 && kChainSteps[0][0] <= kChainSteps[0][1] &&
-                  kChainSteps[1][0] <= kChainSteps[1][1] && mel_vec(0) <= kMelVecMax,
-              "chains are whole float4 steps, chain 1 the longer");
+constexpr int kMelSlots = 2;
+constexpr int kMelSteps[kSchedules][kMelSlots] = {{3, 14}, {4, 20}};
+constexpr int mel_vec(int schedule) { return (kMelSteps[schedule][0] + kMelSteps[schedule][1] + 3) / 4; }
+constexpr int kMelVecMax = mel_vec(1);  // float4 weights per lane, either schedule
+static_assert(mel_vec(0) <= kMelVecMax, "the weight table holds either schedule");
 
 // Raw log-mel (log2; times ln 2 is the log-mel) lives in scratch in tiles
-// of 16 frames (kRawTile floats): 8 slabs of 16 features, each [16 frames]
-// [16 features], slab s holding features 16s..16s+15.  Frame f of a region
-// whose tile 0 holds frames 0..15 sits at region + raw_frame(f).
+// of 16 frames (kRawTile floats): 8 slabs of 16 features, slab s holding
+// features 16 s .. 16 s + 15 as [4 quads][16 features][4 frames], so that the
+// 4 frames of one feature that a log-mel lane computes are 16 bytes.  Frame f
+// of a region whose tile 0 holds frames 0..15 has its slab 0, feature 0 at
+// region + raw_frame(f); feature m of slab s 256 s + 4 m floats on.
 constexpr int kTile = 16;              // frames per raw tile
 constexpr int kRawTile = kTile * 128;  // raw scratch floats per tile of 16 frames
+constexpr int kRawSlab = 256;          // floats per slab of a tile
 constexpr int kQuad = 4;               // frames per unit of work (one wave pass) of the log-mel kernel
-__host__ __device__ constexpr int64_t raw_frame(int64_t f) { return kRawTile * (f >> 4) + 16 * (f & 15); }
+__host__ __device__ constexpr int64_t raw_quad(int64_t q) { return kRawTile * (q >> 2) + 64 * (q & 3); }
+__host__ __device__ constexpr int64_t raw_frame(int64_t f) { return raw_quad(f >> 2) + (f & 3); }
 
 // One entry of either kernel's table.
 //
@@ -67,7 +58,8 @@ __host__ __device__ constexpr int64_t raw_frame(int64_t f) { return kRawTile * (
 // log-mel is read from raw[grid_off + raw_frame(f + gshift)] for f in
 // [f_lo, f_hi], raw[tail_off + raw_frame(f)] past f_hi and raw[out_off +
 // raw_frame(f)] below f_lo.  An item with its own region has f_lo = 0,
-// f_hi = T - 1, grid_off = out_off and gshift = 0.
+// f_hi = T - 1, grid_off = out_off and gshift = 0.  Else f_lo, f_hi + 1 and
+// gshift are multiples of 4: the regions meet at whole quads of the item.
 struct Item {
   int64_t start;
   int64_t len;
@@ -104,9 +96,9 @@ inline Item own_item(int64_t start, int64_t len, int64_t out_off, int64_t dst_of
 }
 
 // Shared frames (sfe_share.cpp).  Frames of overlapping items whose samples
-// lie at least one sample inside each item and whose starts agree modulo the
-// hop are computed once: items' own regions keep only their first quad and
-// their last quads, and a shared log-mel entry per run of such items covers
+// lie at least one sample inside each item and whose starts agree modulo 4
+// hops (one quad) are computed once: items' own regions keep only their first
+// quad and their last quads, and a shared log-mel entry per run of such items covers
 // the union of their interior frames.  Given items with their own regions
 // (own_item; out_off ignored), plan_table fills one table, table[0, *n_lm)
 // with the log-mel entries and table[*n_lm, *n_lm + n) with the
@@ -118,7 +110,7 @@ constexpr int kPlanEntriesPerItem = 3;  // log-mel entries per item at most
 struct PlanWorkspace {
   struct Span {
     int idx;              // item index
-    int64_t res, lo, hi;  // start mod hop; interior frames in recording frame indices
+    int64_t res, lo, hi;  // start mod 4 hops; interior frames in recording frame indices
   };
   struct Run {
     int64_t res, lo, hi;   // union of interior frames (recording frame indices)
@@ -158,29 +150,43 @@ static_assert(kMaxShareFrames * kRawTile / kTile * 4 + (int64_t)kMaxShareMembers
 // Constant tables, uploaded once per context.
 struct DevTables {
   float window[kNfft];       // hann_window(400), zero past 400
-  // Inter-stage twiddles e^{-2 pi i l k1 / 256} (l, k1 < 16) in tangent
-  // form (sfe_fft.hpp tan_twiddle): tan256[l * 16 + k1] = tan, read by lane
-  // l of the first stage; cos256[k1 * 16 + l] = cos, read by lane k1 of the
-  // second stage (dft16_scaled).  At cos = 0 (l k1 = 64): 2^-100 and 2^100.
+  // Inter-stage twiddles e^{-2 pi i k c / 512} (k, c < 16) of the log-mel
+  // kernel's 32 x 16 FFT in tangent form (sfe_fft.hpp tan_twiddle), both
+  // symmetric: tan512[c * 16 + k] is read by lane c of the first stage,
+  // cos512[k * 16 + c] by lane k of the second (dft16_scaled).  Never pi / 2
+  // (k c = 128 needs a factor of 16).
+  float tan512[256];
+  float cos512[256];
+  // Operands of the special columns' MFMAs (the bins that are multiples of
+  // 16): steps 0..3 and 4..7 of lane 4 j + i; see special_bin.
+  float4 special[2][64];
+  // Mel weights: step s of lane L's concatenated slots at mel_w[s / 4][L],
+  // component s % 4; each filter's first bin.
+  float4 mel_w[kMelVecMax][64];
+  int32_t mel_k0[kMelSlots][64];
+  // The same transform as a 16 x 16 complex FFT with an even/odd split
+  // (sfe_fft.hpp dft16_windowed, split_power), which the host check of the
+  // 16-point pieces runs: tan256[l * 16 + k1], cos256[k1 * 16 + l] of
+  // e^{-2 pi i l k1 / 256} (at cos = 0, l k1 = 64: 2^-100 and 2^100), and
+  // split twiddles e^{-2 pi i k / 512}, k < 128, as (cos, tan) for k < 64 and
+  // (sin, cos / sin) above.
   float tan256[256];
   float cos256[256];
-  // Split twiddles e^{-2 pi i k / 512}, k < 128, as (s, r): k < 64: (cos,
-  // tan); k >= 64: (sin, cos / sin) (sfe_fft.hpp split_g).
   float2 split[128];
-  // A operands of the mel MFMAs: [v][lane] holds steps 4v..4v+3 (v < S0 /
-  // 4: chain 0, else chain 1, steps 4(v - S0 / 4)..; S0 = chain 0's steps)
-  // of lane L = 4j + m: filter 64c + 4j + m at bin k0[c][j] + step, times
-  // 0.25 (the FFT stage yields 4|X|^2).  The first mel_vec(schedule) rows
-  // are used.
-  float4 mel_a[kMelVecMax][64];
-  int32_t k0[kChains][16];  // first bin of each block (multiple of 4)
-  int32_t schedule;         // index into kChainSteps
+  int32_t schedule;         // index into kMelSteps
 };
+
+// Special columns of the log-mel kernel's FFT: block j (of 16) sums half j / 8
+// of the inputs of pair q = j % 8; the pair's two bins (h = 0, 1) are
+// multiples of 32 from Y[0] (q < 4) or odd multiples of 16 from Y[16].
+__host__ __device__ constexpr int special_bin(int q, int h) {
+  return q < 4 ? 32 * (2 * q + 1 + h) : 16 + 32 * (2 * (q - 4) + h);
+}
 
 // Host table builders (sfe_tables.cpp).
 void hann_window(int win, float* out);
 void mel_filterbank(int n_fft, int n_mels, int sample_rate, float* out);
-// Returns false if the filterbank does not fit the MFMA schedule.
+// Returns false if the filterbank fits no mel schedule.
 bool build_dev_tables(int sample_rate, DevTables* t);
 
 // Kernel launchers (sfe_kernels.hip).  All asynchronous on `stream`.

@@ -62,6 +62,40 @@ void mel_filterbank(int n_fft, int n_mels, int sample_rate, float* out) {
   }
 }
 
+namespace {
+// Chooses k0[j] in (hi[j] - S, lo[j]] with distinct k0[j] mod 16, as far as a
+// matching (augmenting paths) finds one; the others keep lo[j].
+void spread_banks(const int (&lo)[16], const int (&hi)[16], int S, int (&k0)[16]) {
+  int owner[16];  // bank group -> lane
+  for (int& o : owner) o = -1;
+  struct Search {
+    const int (&lo)[16];
+    const int (&hi)[16];
+    int S;
+    int (&k0)[16];
+    int (&owner)[16];
+    bool seen[16];
+    bool place(int j) {
+      for (int k = lo[j]; k >= 0 && k > hi[j] - S; --k) {
+        const int u = k % 16;
+        if (seen[u]) continue;
+        seen[u] = true;
+        if (owner[u] < 0 || place(owner[u])) {
+          owner[u] = j;
+          k0[j] = k;
+          return true;
+        }
+      }
+      return false;
+    }
+  };
+  for (int j = 0; j < 16; ++j) {
+    Search s{lo, hi, S, k0, owner, {}};
+    s.place(j);
+  }
+}
+}  // namespace
+
 bool build_dev_tables(int sample_rate, DevTables* t) {
   memset(t, 0, sizeof(*t));
   hann_window(kWin, t->window);
@@ -88,47 +122,79 @@ bool build_dev_tables(int sample_rate, DevTables* t) {
     const double b = 2.0 * M_PI * (double)k / 512.0, c = cos(b), s = sin(b);
     t->split[k] = k < 64 ? make_float2((float)c, (float)(s / c)) : make_float2((float)s, (float)(c / s));
   }
+  for (int k = 0; k < 16; ++k)
+    for (int c = 0; c < 16; ++c) {
+      const double th = 2.0 * M_PI * (double)(k * c) / 512.0;
+      t->tan512[k * 16 + c] = (float)(sin(th) / cos(th));
+      t->cos512[k * 16 + c] = (float)cos(th);
+    }
+  for (int L = 0; L < 64; ++L) {
+    // rows i = 0..3 of a block: real and imaginary parts of its two bins
+    const int j = L / 4, i = L % 4, bin = special_bin(j % 8, i / 2);
+    for (int s = 0; s < 8; ++s) {
+      const int m = (bin * (8 * (j / 8) + s)) % 512;  // a multiple of 16
+      const double th = 2.0 * M_PI * (double)m / 512.0;
+      const bool zero = i % 2 == 0 ? m % 256 == 128 : m % 256 == 0;
+      reinterpret_cast<float*>(&t->special[s / 4][L])[s % 4] = zero ? 0.0f : (float)(i % 2 == 0 ? cos(th) : -sin(th));
+    }
+  }
   std::vector<float> fb((size_t)kMel * kBins);
   mel_filterbank(kNfft, kMel, sample_rate, fb.data());
-  // 4-filter blocks: the first bin (a multiple of 4) is chosen here; the
-  // block's nonzero bins must fit its chain's step count, and every bin
-  // read must lie within the bins the FFT stage writes (kBinsWritten).  The
-  // first schedule every block fits is used.
-  auto fill = [&](int sch) -> bool {
-    for (int c = 0; c < kChains; ++c) {
-      const int S = kChainSteps[sch][c];
-      for (int j = 0; j < 16; ++j) {
-        const int f0 = 64 * c + 4 * j;
-        int lo = -1, hi = -1;
-        for (int m = f0; m < f0 + 4; ++m)
-          for (int k = 0; k < kBins; ++k)
-            if (fb[(size_t)m * kBins + k] != 0.0f) {
-              if (lo < 0 || k < lo) lo = k;
-              if (k > hi) hi = k;
-            }
-        if (lo < 0) lo = hi = 0;
-        int k0 = lo / 4 * 4;
-        if (k0 + S > kBinsWritten[sch]) k0 = (kBinsWritten[sch] - S) / 4 * 4;
-        if (lo < k0 || hi >= k0 + S) return false;  // filters too wide for this schedule
-        t->k0[c][j] = k0;
-        for (int s = 0; s < S; ++s)
-          for (int m = 0; m < 4; ++m) {
-            const int v = (c == 0 ? 0 : kChainSteps[sch][0] / 4) + s / 4;
-            float* a = reinterpret_cast<float*>(&t->mel_a[v][4 * j + m]);
-            a[s % 4] = fb[(size_t)(f0 + m) * kBins + k0 + s] * 0.25f;
+  // The sample rates taken and their schedule follow from the band edges of
+  // blocks of 4 filters: from a first bin that is a multiple of 4, the blocks
+  // of filters 0..63 span at most 8 bins and those of 64..127 at most 32
+  // (schedule 0), or 12 and 48 (schedule 1, which may also run 3 bins past
+  // the spectrum).  Rates outside are refused; the slots of kMelSteps hold
+  // every filter of those inside.
+  auto fits = [&](int low, int high, int bins) -> bool {
+    for (int f0 = 0; f0 < kMel; f0 += 4) {
+      const int S = f0 < 64 ? low : high;
+      int lo = -1, hi = -1;
+      for (int m = f0; m < f0 + 4; ++m)
+        for (int k = 0; k < kBins; ++k)
+          if (fb[(size_t)m * kBins + k] != 0.0f) {
+            if (lo < 0 || k < lo) lo = k;
+            if (k > hi) hi = k;
           }
-      }
+      if (lo < 0) lo = hi = 0;
+      int k0 = lo / 4 * 4;
+      if (k0 + S > bins) k0 = (bins - S) / 4 * 4;
+      if (lo < k0 || hi >= k0 + S) return false;
     }
-    t->schedule = sch;
     return true;
   };
-  bool ok = false;
-  for (int sch = 0; sch < kSchedules && !ok; ++sch) {
-    memset(t->mel_a, 0, sizeof(t->mel_a));
-    memset(t->k0, 0, sizeof(t->k0));
-    ok = fill(sch);
+  if (fits(8, 32, kBins)) t->schedule = 0;
+  else if (fits(12, 48, kBins + 3)) t->schedule = 1;
+  else return false;
+  int first = 0;  // steps before the slot's
+  for (int i = 0; i < kMelSlots; ++i) {
+    const int S = kMelSteps[t->schedule][i];
+    for (int g = 0; g < 64; g += 16) {
+      int lo[16], hi[16], k0[16];
+      for (int j = 0; j < 16; ++j) {
+        const float* f = &fb[(size_t)(64 * i + g + j) * kBins];
+        lo[j] = 0, hi[j] = kBins - 1;
+        while (lo[j] < kBins && f[lo[j]] == 0.0f) ++lo[j];
+        while (hi[j] > lo[j] && f[hi[j]] == 0.0f) --hi[j];
+        if (lo[j] == kBins) lo[j] = hi[j] = 0;  // an all-zero filter
+        lo[j] = std::min(lo[j], kBins - S);
+        if (hi[j] >= lo[j] + S) return false;
+        k0[j] = lo[j];
+      }
+      // 16 lanes' 16-byte reads of power bins fall on 16 groups of banks:
+      // slot 1's filters are wider apart than the first bins of slot 0's,
+      // which mostly share bins, so where the slot is wider than the filter
+      // its first bin is moved down to spread them.
+      if (i == 1) spread_banks(lo, hi, S, k0);
+      for (int j = 0; j < 16; ++j) {
+        const float* f = &fb[(size_t)(64 * i + g + j) * kBins];
+        t->mel_k0[i][g + j] = k0[j];
+        for (int s = 0; s < S; ++s)
+          reinterpret_cast<float*>(&t->mel_w[(first + s) / 4][g + j])[(first + s) % 4] = f[k0[j] + s];
+      }
+    }
+    first += S;
   }
-  if (!ok) return false;
   return true;
 }
 

@@ -200,6 +200,7 @@ struct sfe_ctx {
   hipStream_t last_stream = nullptr;  // the stream the previous call's device work ran on
   PinBuf h_meta;
   DevBuf scratch;   // raw log-mel in 16-frame tiles, f32 (the normalisation kernel's input)
+  DevBuf parts;     // partial sums of long items' segments (sfe::launch_norm)
   DevBuf io_in;     // sfe_extract staging (audio)
   DevBuf io_out;    // sfe_extract staging (features)
   PinBuf h_io_in;   // sfe_extract pinned host staging: copies of pageable
@@ -219,6 +220,7 @@ struct sfe_ctx {
   std::vector<Item> plan_table;
   size_t plan_n_lm = 0;
   int64_t plan_tiles = 0;
+  int64_t plan_segs = 0;  // segments of the long items
   // kernel timing (sfe_set_timing): events around each launch, summed on read
   bool timing = false;
   std::vector<hipEvent_t> tev;  // pairs: start, end; kind alternates logmel, norm
@@ -310,9 +312,16 @@ hipEvent_t timing_event(sfe_ctx* ctx) {
 // bandwidth from it.)
 enum Stages { kLogmel = 1, kNorm = 2, kBoth = 3 };
 
+// Long items of a normalisation launch (sfe::norm_segments).
+struct Segments {
+  int n = 0;
+  const int32_t* d_item = nullptr;
+  void* parts = nullptr;
+};
+
 int launch_pair(sfe_ctx* ctx, const Source& src, const Item* lm, const Item* d_lm, int n_lm, const Item* norm,
-                const Item* d_norm, int n_norm, float* raw, void* out, int32_t out_dtype, int pad_to,
-                hipStream_t stream, int stages = kBoth, bool allow_timing = true,
+                const Item* d_norm, int n_norm, const Segments& segs, float* raw, void* out, int32_t out_dtype,
+                int pad_to, hipStream_t stream, int stages = kBoth, bool allow_timing = true,
                 const int32_t* d_wave_item = nullptr) {
   if (n_lm <= 0 && n_norm <= 0) return SFE_OK;
   const int u0 = n_lm > 0 ? lm[0].unit_off : 0;
@@ -330,7 +339,8 @@ int launch_pair(sfe_ctx* ctx, const Source& src, const Item* lm, const Item* d_l
   if (e[1]) SFE_HIP(hipEventRecord(e[1], stream));
   if (e[2]) SFE_HIP(hipEventRecord(e[2], stream));
   if (stages & kNorm)
-    SFE_HIP(sfe::launch_norm(raw, d_norm, n_norm, max_T, pad_to, out, out_dtype == SFE_BF16, stream));
+    SFE_HIP(sfe::launch_norm(raw, d_norm, n_norm, max_T, pad_to, out, out_dtype == SFE_BF16, segs.n, segs.d_item,
+                             segs.parts, stream));
   if (e[3]) SFE_HIP(hipEventRecord(e[3], stream));
   return SFE_OK;
 }
@@ -369,6 +379,8 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
     ctx->plan_tiles = sfe::plan_table(items.data(), n, ctx->share, &ws, table.data(), &n_lm);
     sfe::order_norm(table.data() + n_lm, n);
     table.resize(n_lm + items.size());
+    ctx->plan_segs = sfe::norm_segments(table.data() + n_lm, n, nullptr);
+    if (ctx->plan_segs > INT32_MAX / 8) return fail(SFE_INVALID_ARG, "batch too large for one launch");
     ctx->plan_n_lm = n_lm;
     ctx->plan_table.swap(table);
     ctx->plan_in = items;
@@ -377,13 +389,15 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
   const std::vector<Item>& table = ctx->plan_table;
   const size_t n_lm = ctx->plan_n_lm;
   const int64_t total_tiles = ctx->plan_tiles;
-  // The upload: the table, then the log-mel launch's first-item table.
+  // The upload: the table, then the log-mel launch's first-item table, then
+  // the long items' segments.
   const size_t tbytes = table.size() * sizeof(Item);
   const WaveTable wt = wave_table(table.data(), n_lm, ctx->cus);
-  const size_t mbytes = tbytes + wt.entries * sizeof(int32_t);
+  const size_t sbytes = tbytes + wt.entries * sizeof(int32_t);
+  const size_t mbytes = sbytes + (size_t)ctx->plan_segs * sizeof(int32_t);
   // A call with the same table as the previous upload (repeated plans,
   // equal-sized windows) reuses the device copy (the first-item table
-  // follows from the table).  The table is only read by the kernels, so
+  // and the segments follow from the table).  The table is only read by the kernels, so
   // earlier work still in flight is unaffected.
   const bool same = ctx->meta.ptr && ctx->meta_items.size() == table.size() &&
                     memcmp(ctx->meta_items.data(), table.data(), tbytes) == 0;
@@ -395,6 +409,9 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
     if (wt.entries)
       sfe::logmel_wave_items(table.data(), (int)n_lm, wt.u0, wt.n_units, wt.grid,
                              reinterpret_cast<int32_t*>(static_cast<char*>(ctx->h_meta.ptr) + tbytes));
+    if (ctx->plan_segs > 0)
+      sfe::norm_segments(ctx->plan_table.data() + n_lm, (int)items.size(),
+                         reinterpret_cast<int32_t*>(static_cast<char*>(ctx->h_meta.ptr) + sbytes));
     SFE_HIP(hipMemcpyAsync(ctx->meta.ptr, ctx->h_meta.ptr, mbytes, hipMemcpyHostToDevice, stream));
     SFE_HIP(hipEventRecord(ctx->h_meta.ev, stream));
     ctx->h_meta.pending = true;
@@ -404,9 +421,13 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
   const int32_t* d_wave =
       wt.entries ? reinterpret_cast<const int32_t*>(static_cast<const char*>(ctx->meta.ptr) + tbytes) : nullptr;
   SFE_HIP(ctx->scratch.reserve((size_t)total_tiles * sfe::kRawTile * sizeof(float)));
+  SFE_HIP(ctx->parts.reserve((size_t)ctx->plan_segs * sfe::kSegPartBytes));
   float* raw = static_cast<float*>(ctx->scratch.ptr);
+  const Segments segs{(int)ctx->plan_segs,
+                      reinterpret_cast<const int32_t*>(static_cast<const char*>(ctx->meta.ptr) + sbytes),
+                      ctx->parts.ptr};
   const int rc = launch_pair(ctx, src, table.data(), d_table, (int)n_lm, table.data() + n_lm, d_table + n_lm,
-                             (int)items.size(), raw, out, out_dtype, pad_to, stream, kBoth, true, d_wave);
+                             (int)items.size(), segs, raw, out, out_dtype, pad_to, stream, kBoth, true, d_wave);
   if (rc) return rc;
   SFE_HIP(mark_last(ctx, stream));
   return SFE_OK;
@@ -614,6 +635,7 @@ void sfe_destroy(sfe_ctx* ctx) {
   ctx->meta.release();
   ctx->h_meta.release();
   ctx->scratch.release();
+  ctx->parts.release();
   ctx->io_in.release();
   ctx->io_out.release();
   ctx->h_io_in.release();
@@ -825,7 +847,8 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
       SFE_HIP(sfe::noalloc_scratch(ctx->device, &na));
       ctx->noalloc = static_cast<unsigned char*>(na);
     }
-    if (ctx->h_meta.cap < entries * sizeof(Item) + sfe::kMaxLogmelWaves * sizeof(int32_t) ||
+    if (ctx->h_meta.cap <
+            entries * sizeof(Item) + (sfe::kMaxLogmelWaves + sfe::kNoAllocMaxSegs) * sizeof(int32_t) ||
         ctx->na_in.capacity() < (size_t)n)
       return fail(SFE_HIP_ERROR, "context has no reserved planner buffers");
     int64_t fo = 0, own_tiles = 0;
@@ -847,12 +870,15 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
     tiles = sfe::plan_table(ctx->na_in.data(), n, share, &ctx->na_ws, table, &n_lm);
     if (share && tiles > own_tiles) tiles = sfe::plan_table(ctx->na_in.data(), n, false, &ctx->na_ws, table, &n_lm);
     sfe::order_norm(table + n_lm, n);
+    const int64_t n_segs = sfe::norm_segments(table + n_lm, n, nullptr);
+    if (n_segs > sfe::kNoAllocMaxSegs) return fail(SFE_HIP_ERROR, "segments outgrow the static scratch");
     SFE_HIP(order_after_last(ctx, s));
     SFE_HIP(sfe::noalloc_order(ctx->device, s));
     Item* d_table = reinterpret_cast<Item*>(ctx->noalloc);
     float* raw = reinterpret_cast<float*>(ctx->noalloc + sfe::kNoAllocItemBytes);
-    // the table, then the log-mel launch's first-item table, in one copy
-    // (the item region holds kMaxLogmelWaves entries past the largest table)
+    // the table, then the log-mel launch's first-item table and the long
+    // items' segments, in one copy (the item region holds kMaxLogmelWaves +
+    // kNoAllocMaxSegs entries past the largest table)
     const size_t tbytes = (n_lm + n) * sizeof(Item);
     const WaveTable wt = wave_table(table, n_lm, ctx->cus);
     if (wt.entries)
@@ -860,10 +886,15 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
                              reinterpret_cast<int32_t*>(reinterpret_cast<char*>(table) + tbytes));
     const int32_t* d_wave =
         wt.entries ? reinterpret_cast<const int32_t*>(ctx->noalloc + tbytes) : nullptr;
-    SFE_HIP(hipMemcpyAsync(d_table, table, tbytes + wt.entries * sizeof(int32_t), hipMemcpyHostToDevice, s));
+    const size_t sbytes = tbytes + wt.entries * sizeof(int32_t);
+    if (n_segs > 0)
+      sfe::norm_segments(table + n_lm, n, reinterpret_cast<int32_t*>(reinterpret_cast<char*>(table) + sbytes));
+    const Segments segs{(int)n_segs, reinterpret_cast<const int32_t*>(ctx->noalloc + sbytes),
+                        ctx->noalloc + sfe::kNoAllocItemBytes + sfe::kNoAllocRawBytes};
+    SFE_HIP(hipMemcpyAsync(d_table, table, sbytes + (size_t)n_segs * sizeof(int32_t), hipMemcpyHostToDevice, s));
     SFE_HIP(hipEventRecord(ctx->h_meta.ev, s));
     ctx->h_meta.pending = true;
-    rc = launch_pair(ctx, f32_source(recording), table, d_table, (int)n_lm, table + n_lm, d_table + n_lm, n, raw, out,
+    rc = launch_pair(ctx, f32_source(recording), table, d_table, (int)n_lm, table + n_lm, d_table + n_lm, n, segs, raw, out,
                      out_dtype, 0, s, kBoth, false, d_wave);
     if (rc) return rc;
     SFE_HIP(mark_last(ctx, s));
@@ -1064,47 +1095,77 @@ int sfe_extract_chunks_streamed_pcm(sfe_ctx* ctx, const void* host_recording, in
       }
       tiles = raw_tiles;
     }
+    // Normalisation reads only the raw log-mel (all of it stays in HBM), so
+    // it runs once per kStreamNormWindows windows or more instead of per
+    // batch: one launch over many items instead of many launches over a few.
+    // A group of batches is normalised after its last batch; its long items'
+    // segments are entries [seg0, seg0 + n_segs) of the uploaded list.
+    struct NormGroup {
+      size_t last;  // batch
+      int32_t first, end;
+      int64_t seg0, n_segs;
+    };
+    std::vector<NormGroup> norm_groups;
+    int64_t total_segs = 0, max_segs = 0;
+    {
+      int32_t first = 0;
+      size_t windows = 0;
+      for (size_t bi = 0; bi < batches.size(); ++bi) {
+        windows += batches[bi].g1 - batches[bi].g0;
+        if (bi + 1 < batches.size() && windows < kStreamNormWindows) continue;
+        const Group& g = groups[batches[bi].g1 - 1];
+        const int32_t end = g.first + g.count;
+        const int64_t k = sfe::norm_segments(nm_tab.data() + first, end - first, nullptr);
+        norm_groups.push_back({bi, first, end, total_segs, k});
+        total_segs += k;
+        max_segs = std::max(max_segs, k);
+        first = end;
+        windows = 0;
+      }
+    }
+    if (max_segs > INT32_MAX / 8) return fail(SFE_INVALID_ARG, "batch too large for one launch");
     const size_t n_lm_all = lm_tab.size();
     lm_tab.insert(lm_tab.end(), nm_tab.begin(), nm_tab.end());
     const std::vector<Item>& table = lm_tab;  // log-mel entries, then normalisation entries
-    const size_t mbytes = table.size() * sizeof(Item);
+    const size_t tbytes = table.size() * sizeof(Item);
+    const size_t mbytes = tbytes + (size_t)total_segs * sizeof(int32_t);
     ctx->meta_items.clear();  // the table uploaded below is re-based per window group
     SFE_HIP(ctx->h_meta.reserve(mbytes));
     SFE_HIP(ctx->meta.reserve(mbytes));
     SFE_HIP(ctx->scratch.reserve((size_t)tiles * sfe::kRawTile * sizeof(float)));
+    SFE_HIP(ctx->parts.reserve((size_t)max_segs * sfe::kSegPartBytes));
     float* raw = static_cast<float*>(ctx->scratch.ptr);
-    memcpy(ctx->h_meta.ptr, table.data(), mbytes);
+    memcpy(ctx->h_meta.ptr, table.data(), tbytes);
+    int32_t* seg_list = reinterpret_cast<int32_t*>(static_cast<char*>(ctx->h_meta.ptr) + tbytes);
+    for (const NormGroup& g : norm_groups)
+      if (g.n_segs > 0) sfe::norm_segments(nm_tab.data() + g.first, g.end - g.first, seg_list + g.seg0);
     SFE_HIP(hipMemcpyAsync(ctx->meta.ptr, ctx->h_meta.ptr, mbytes, hipMemcpyHostToDevice, sc));
     SFE_HIP(hipEventRecord(ctx->h_meta.ev, sc));
     ctx->h_meta.pending = true;
     const Item* d_items = static_cast<const Item*>(ctx->meta.ptr);
     Source rsrc = src;
     rsrc.ptr = ring;
-    int32_t norm_first = 0;
-    size_t norm_windows = 0;  // windows featurized since the last normalisation
+    size_t next_norm = 0;  // group
     for (size_t bi = 0; bi < batches.size(); ++bi) {
       const Batch& bt = batches[bi];
       const int e = (int)(bi & 1);
       if (bi > 0 && (rc = issue_copy(bi))) return rc;
       SFE_HIP(hipStreamWaitEvent(sc, ctx->ev_copied[e], 0));
-      const int32_t end = groups[bt.g1 - 1].first + groups[bt.g1 - 1].count;
       const Item* lm = table.data() + lm_at[bi];
       const int n_lm = (int)(lm_at[bi + 1] - lm_at[bi]);
-      rc = launch_pair(ctx, rsrc, lm, d_items + lm_at[bi], n_lm, nullptr, nullptr, 0, raw, out, out_dtype, 0, sc,
-                       kLogmel);
+      rc = launch_pair(ctx, rsrc, lm, d_items + lm_at[bi], n_lm, nullptr, nullptr, 0, Segments{}, raw, out, out_dtype,
+                       0, sc, kLogmel);
       if (rc) return rc;
       SFE_HIP(hipEventRecord(ctx->ev_done[e], sc));
-      // Normalisation reads only the raw log-mel (all of it stays in HBM), so
-      // it runs once per kStreamNormWindows windows or more instead of per
-      // batch: one launch over many items instead of many launches over a few.
-      norm_windows += bt.g1 - bt.g0;
-      if (bi + 1 == batches.size() || norm_windows >= kStreamNormWindows) {
-        const size_t nf = n_lm_all + (size_t)norm_first;
-        rc = launch_pair(ctx, rsrc, nullptr, nullptr, 0, table.data() + nf, d_items + nf, end - norm_first, raw, out,
-                         out_dtype, 0, sc, kNorm);
+      if (norm_groups[next_norm].last == bi) {
+        const NormGroup& g = norm_groups[next_norm++];
+        const size_t nf = n_lm_all + (size_t)g.first;
+        const Segments segs{(int)g.n_segs,
+                            reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(d_items) + tbytes) + g.seg0,
+                            ctx->parts.ptr};
+        rc = launch_pair(ctx, rsrc, nullptr, nullptr, 0, table.data() + nf, d_items + nf, g.end - g.first, segs, raw,
+                         out, out_dtype, 0, sc, kNorm);
         if (rc) return rc;
-        norm_first = end;
-        norm_windows = 0;
       }
     }
     SFE_HIP(hipStreamSynchronize(sc));

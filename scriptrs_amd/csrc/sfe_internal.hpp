@@ -72,7 +72,7 @@ struct Item {
   int32_t n_units;   // log-mel: units of the entry
   int32_t q0;        // log-mel: first quad of the entry within its frames
   int32_t f_lo, f_hi, gshift;
-  int32_t pad_;
+  int32_t seg0;      // normalisation: first segment of a long item (norm_segments)
 };
 static_assert(sizeof(Item) == 80, "item table layout");
 
@@ -134,6 +134,27 @@ int64_t plan_table(const Item* items, int n, bool share, PlanWorkspace* ws, Item
 // Normalisation entries reordered longest first (in 256-frame classes, call
 // order within one); allocates nothing.
 void order_norm(Item* norm, int n);
+// Long items (more than kNormRegFrames frames, what a normalisation workgroup
+// holds in registers) are normalised in segments of seg_frames(T) frames, at
+// most 64 an item (sfe_kernels.hip norm_segment).  norm_segments numbers the
+// segments of table entries norm[0, n) (Item::seg0), writes each segment's
+// entry index to seg_item unless it is null, and returns their count.  A
+// segment leaves kSegPartBytes of partial sums.
+constexpr int kNormRegFrames = 2048;
+constexpr int kSegFrames = 512;
+constexpr int kSegPartBytes = kMel * 2 * (int)sizeof(double);
+__host__ __device__ constexpr int seg_frames(int T) { return kSegFrames * ((T - 1) / (64 * kSegFrames) + 1); }
+inline int64_t norm_segments(Item* norm, int n, int32_t* seg_item) {
+  int64_t segs = 0;
+  for (int i = 0; i < n; ++i) {
+    if (norm[i].T <= kNormRegFrames) continue;
+    norm[i].seg0 = (int32_t)segs;
+    const int k = (norm[i].T - 1) / seg_frames(norm[i].T) + 1;
+    for (int s = 0; s < k && seg_item; ++s) seg_item[segs + s] = i;
+    segs += k;
+  }
+  return segs;
+}
 // Frames of one run's shared entry at most (512 MB of raw log-mel), and
 // members of one run at most (each with at most 3 tiles of its own, 384 MB
 // in all): an item's first and last tiles follow its run's shared region,
@@ -257,20 +278,26 @@ hipError_t launch_logmel(const void* samples, int pcm, float pcm_scale, const It
 // and writes feature-major [128][T] per item to out (f32, must not alias
 // raw) or bf16 (uint16_t*) when out_bf16 is set.  max_T: the longest item's
 // frame count (sizes the kernel's register budget).  pad_to > 0: rows of
-// pad_to frames, zero past T (the encoder input layout).
+// pad_to frames, zero past T (the encoder input layout).  n_segs, seg_item,
+// parts: the long items' segments (norm_segments over items), the device copy
+// of their entry indexes and n_segs * kSegPartBytes of scratch.
 hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int pad_to, void* out,
-                       bool out_bf16, hipStream_t stream);
+                       bool out_bf16, int n_segs, const int32_t* seg_item, void* parts, hipStream_t stream);
 
 // Static scratch of the allocation-free entry point (sfe_noalloc.hip): an
 // item table of up to kNoAllocMaxItems items, then kNoAllocRawBytes of raw
-// log-mel (kNoAllocRawBytes / (kRawTile * 4) 16-frame tiles).
+// log-mel (kNoAllocRawBytes / (kRawTile * 4) 16-frame tiles), then the partial
+// sums of long items.
 constexpr int kNoAllocMaxItems = 4096;
 // (a plan has at most kPlanEntriesPerItem log-mel entries and one
 // normalisation entry per item)
-constexpr size_t kNoAllocItemBytes =
-    ((size_t)(kPlanEntriesPerItem + 1) * kNoAllocMaxItems * sizeof(Item) + kMaxLogmelWaves * sizeof(int32_t) +
-     255) / 256 * 256;
 constexpr size_t kNoAllocRawBytes = (size_t)64 << 20;
+// Segments of long items within that much raw log-mel: each item's last one
+// may be short, and a long item has more than 4.
+constexpr int kNoAllocMaxSegs = (int)(kNoAllocRawBytes / (kRawTile * 4) * kTile / kSegFrames * 5 / 4) + 1;
+constexpr size_t kNoAllocItemBytes = ((size_t)(kPlanEntriesPerItem + 1) * kNoAllocMaxItems * sizeof(Item) +
+                                      (kMaxLogmelWaves + kNoAllocMaxSegs) * sizeof(int32_t) + 255) / 256 * 256;
+constexpr size_t kNoAllocPartBytes = (size_t)kNoAllocMaxSegs * kSegPartBytes;
 // Device address of this device's static scratch (looked up once per device).
 hipError_t noalloc_scratch(int device, void** out);
 // Host lock of a device's static scratch (held for a whole call), and the

@@ -528,7 +528,7 @@ __device__ __forceinline__ void constant_row_stats(float x0, int T, float* mean_
 // j, lane i of wave v holds the 4 frames of quad 4 (W j + v) + i / 16 of
 // feature i % 16, one float4, and a wave's load is 1 KB of one raw tile.
 // Items of up to 16 W N frames are read from HBM once and held in registers
-// (N float4s per lane); longer ones are streamed three times.  Stores: chunks
+// (N float4s per lane); longer ones go in segments (norm_segment).  Stores: chunks
 // of 4 rounds are transposed through LDS and each lane writes 4 consecutive
 // frames of one feature row, so a store instruction covers 16 / W rows of
 // contiguous bytes (rows are only 4-byte aligned when T is odd; gfx950 takes
@@ -543,7 +543,6 @@ __device__ __forceinline__ void constant_row_stats(float x0, int T, float* mean_
 // reference).  A feature whose values are all equal (squared deviations that
 // sum to exactly 0: the f32 mean is then that value) replays the reference's
 // sequential f32 sums (constant_row_stats).
-constexpr int kNormBatch = 8;  // rounds of loads in flight on the streaming path
 constexpr int kSlabF = 16;  // features per slab
 constexpr int kSlabs = kMel / kSlabF;
 // Fourth word of a raw buffer resource (no format conversion, no swizzle).
@@ -593,10 +592,11 @@ __device__ __forceinline__ float row_mean(float x0, double S, int T) { return (f
 // Per-feature (mean, sd, 1/sd) of the slab, published in LDS for the store
 // phase by wave 0's lanes 0..15, one feature each.  S: sum of (x - x0), Q:
 // sum of squared deviations from the f32 mean.
-__device__ __forceinline__ void publish_stats(double S, double Q, float x0, int T, int lane, int w, float* st) {
+__device__ __forceinline__ void publish_stats(double S, double Q, bool constant, float x0, int T, int lane, int w,
+                                              float* st) {
   if (w == 0 && lane < kSlabF) {
     float mean, sd;
-    if (Q == 0.0) {
+    if (constant) {
       constant_row_stats(x0, T, &mean, &sd);
     } else {
       mean = row_mean(x0, S, T);
@@ -655,8 +655,9 @@ __device__ __forceinline__ void zero_tail(O* __restrict__ ob, int T, int rs, int
 }
 
 // Where a normalisation workgroup's lane finds its quads: round j holds quad
-// q + 4 W j of the item, at byte off(j) from the uniform base (the start of
-// the item's shared frames, this slab).  An item's own first quad and last
+// q + 4 W j of the item (q counts from quad q0, a multiple of 4, where the
+// workgroup starts), at byte off(j) from the uniform base (the tile of the
+// item's shared frames where the workgroup starts, this slab).  An item's own first quad and last
 // tiles come after its shared region (at most kMaxShareFrames frames, then at
 // most 3 tiles for each of at most kMaxShareMembers members), so 32-bit byte
 // offsets reach them; an item with its own region has all three at out_off.
@@ -671,11 +672,12 @@ struct Rounds {
   int left;      // T - 4 q: element e of round j is inside the item where 16 W j + e < left
   static constexpr uint32_t kRound = 4u * kRawTile * W;  // bytes
 
-  __device__ __forceinline__ Rounds(const float* raw, const Item& it, int slab, int lane, int w) {
-    base = reinterpret_cast<const char*>(raw + it.grid_off + kRawSlab * slab);
-    q = 4 * w + (lane >> 4);
+  __device__ __forceinline__ Rounds(const float* raw, const Item& it, int slab, int lane, int w, int q0) {
     const int gs = it.gshift / kQuad;
-    og = 4u * (uint32_t)(raw_quad(q + gs) + 4 * (lane & 15));
+    const int tile0 = (q0 + gs) & ~3;  // quad of the shared region at the base: offsets stay small in any item
+    base = reinterpret_cast<const char*>(raw + it.grid_off + raw_quad(tile0) + kRawSlab * slab);
+    q = q0 + 4 * w + (lane >> 4);
+    og = 4u * (uint32_t)(raw_quad(q + gs - tile0) + 4 * (lane & 15));
     const int64_t own = raw_quad(q) - raw_quad(q + gs) - it.grid_off;
     dlo = 4u * (uint32_t)(it.out_off + own);
     dhi = 4u * (uint32_t)(it.tail_off + own);
@@ -693,8 +695,12 @@ struct Rounds {
   __device__ __forceinline__ int buf_off(int j) const {
     return 16 * W * j < left ? (int)off(j) : kNormBufRange;
   }
-  // Whether every lane of the workgroup holds 4 frames of the item in round j.
+  // Whether every lane of the workgroup holds 4 frames of the item in round j,
+  // T frames counted from the workgroup's first.
   static __device__ __forceinline__ bool full(int j, int T) { return 16 * W * (j + 1) <= T; }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer() const {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, kNormBufRange, kBufWord3);
+  }
 };
 
 // Adds the f32 sum over a quad of (x - p) to s; elements past the item (index >= n)
@@ -727,10 +733,10 @@ __device__ __forceinline__ void add_sq(double& s, const float4& v, float p, bool
   asm volatile("" : "+v"(s));
 }
 
-// W waves, N float4 registers per lane: items of up to 16 W N frames are held
-// in registers and read once, longer items take the streaming path (three
-// passes).  Every path sums the same quads, so the class does not change the
-// result.  `work` is the (item, slab) index.
+// W waves, N float4 registers per lane: an item of up to 16 W N frames, held
+// in registers and read once.  Every N sums the same quads, so the class does
+// not change the result.  `work` is the (item, slab) index; items longer than
+// kNormRegFrames are left to norm_segment and norm_finish.
 template <int W, int N, typename O>
 __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const Item* __restrict__ items,
                                           int n_items, int work, int pad_to, O* __restrict__ out) {
@@ -757,7 +763,8 @@ __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const I
   const int slab = work % kSlabs;
   const Item it = items[item];
   const int T = it.T;
-  const Rounds<W> rd(raw, it, slab, lane, w);
+  if (T > kNormRegFrames) return;
+  const Rounds<W> rd(raw, it, slab, lane, w, 0);
   const int rs = pad_to > 0 ? pad_to : T;  // output row length
   O* ob = out + it.dst_off + (size_t)(kSlabF * slab) * rs;
   if (pad_to > 0) zero_tail<W>(ob, T, rs, lane, w);
@@ -771,91 +778,40 @@ __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const I
   const int chunks = (T + kChunk - 1) / kChunk;
 
   double s = 0.0, sq = 0.0;
-  if (T <= kSpan * N) {
-    float4 v[N];
-    // Raw buffer loads from the uniform base, all issued before any is used
-    // (a load under a per-lane branch would wait for itself).
-    const __amdgpu_buffer_rsrc_t rsrc =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(rd.base), 0, kNormBufRange, kBufWord3);
+  float4 v[N];
+  // Raw buffer loads from the uniform base, all issued before any is used
+  // (a load under a per-lane branch would wait for itself).
+  const __amdgpu_buffer_rsrc_t rsrc = rd.buffer();
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-      v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
+  for (int j = 0; j < N; ++j)
+    v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      v[j] = ln2_scale(v[j]);
-      add_dev(s, v[j], x0, Rounds<W>::full(j, T), rd.left - kSpan * j);
-    }
-    s = slab_sum<W>(s, red, lane, w);
-#ifdef SFE_TIMESTAMPS
-    if (threadIdx.x == 0) SFE_STAMP(sn + 1, stamp_now());
-#endif
-    const float m = row_mean(x0, s, T);
-#pragma unroll
-    for (int j = 0; j < N; ++j) add_sq(sq, v[j], m, Rounds<W>::full(j, T), rd.left - kSpan * j);
-    sq = slab_sum<W>(sq, red, lane, w);
-    publish_stats(s, sq, x0, T, lane, w, st);
-#ifdef SFE_TIMESTAMPS
-    if (threadIdx.x == 0) SFE_STAMP(sn + 2, stamp_now());
-#endif
-#pragma unroll
-    for (int ch = 0; ch < N / 4; ++ch) {
-      if (ch < chunks) {
-        float* t = tb[ch % kTBufs];
-#pragma unroll
-        for (int jr = 0; jr < 4; ++jr) stage(t, jr, v[4 * ch + jr]);
-        __syncthreads();
-        store_chunk<W>(t, st, kChunk * ch, T, rs, lane, w, ob);
-        if (kTBufs == 1) __syncthreads();
-      }
-    }
-#ifdef SFE_TIMESTAMPS
-    if (threadIdx.x == 0) SFE_STAMP(sn + 3, stamp_now());
-#endif
-    return;
-  }
-
-  // Streaming: three passes over the item, kNormBatch rounds of loads in
-  // flight per lane (the second and third passes mostly hit the caches).
-  constexpr int G = kNormBatch;
-  const int nr = (T + kSpan - 1) / kSpan;
-  auto load = [&](int j) {  // (past the item: the base's first quad, unused)
-    const uint32_t o = kSpan * j < rd.left ? rd.off(j) : 0u;
-    return ln2_scale(*reinterpret_cast<const float4*>(rd.base + o));
-  };
-  for (int j0 = 0; j0 < nr; j0 += G) {
-    float4 e[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) e[g] = load(j0 + g);
-#pragma unroll
-    for (int g = 0; g < G; ++g) add_dev(s, e[g], x0, Rounds<W>::full(j0 + g, T), rd.left - kSpan * (j0 + g));
+  for (int j = 0; j < N; ++j) {
+    v[j] = ln2_scale(v[j]);
+    add_dev(s, v[j], x0, Rounds<W>::full(j, T), rd.left - kSpan * j);
   }
   s = slab_sum<W>(s, red, lane, w);
 #ifdef SFE_TIMESTAMPS
   if (threadIdx.x == 0) SFE_STAMP(sn + 1, stamp_now());
 #endif
   const float m = row_mean(x0, s, T);
-  for (int j0 = 0; j0 < nr; j0 += G) {
-    float4 e[G];
 #pragma unroll
-    for (int g = 0; g < G; ++g) e[g] = load(j0 + g);
-#pragma unroll
-    for (int g = 0; g < G; ++g) add_sq(sq, e[g], m, Rounds<W>::full(j0 + g, T), rd.left - kSpan * (j0 + g));
-  }
+  for (int j = 0; j < N; ++j) add_sq(sq, v[j], m, Rounds<W>::full(j, T), rd.left - kSpan * j);
   sq = slab_sum<W>(sq, red, lane, w);
-  publish_stats(s, sq, x0, T, lane, w, st);
+  publish_stats(s, sq, sq == 0.0, x0, T, lane, w, st);
 #ifdef SFE_TIMESTAMPS
   if (threadIdx.x == 0) SFE_STAMP(sn + 2, stamp_now());
 #endif
-  for (int ch = 0; ch < chunks; ++ch) {
-    float4 e[4];
 #pragma unroll
-    for (int jr = 0; jr < 4; ++jr) e[jr] = load(4 * ch + jr);
-    float* t = tb[ch % kTBufs];
+  for (int ch = 0; ch < N / 4; ++ch) {
+    if (ch < chunks) {
+      float* t = tb[ch % kTBufs];
 #pragma unroll
-    for (int jr = 0; jr < 4; ++jr) stage(t, jr, e[jr]);
-    __syncthreads();
-    store_chunk<W>(t, st, kChunk * ch, T, rs, lane, w, ob);
-    if (kTBufs == 1) __syncthreads();
+      for (int jr = 0; jr < 4; ++jr) stage(t, jr, v[4 * ch + jr]);
+      __syncthreads();
+      store_chunk<W>(t, st, kChunk * ch, T, rs, lane, w, ob);
+      if (kTBufs == 1) __syncthreads();
+    }
   }
 #ifdef SFE_TIMESTAMPS
   if (threadIdx.x == 0) SFE_STAMP(sn + 3, stamp_now());
@@ -871,6 +827,136 @@ __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_kernel(const flo
                                                                        const Item* __restrict__ items, int n_items,
                                                                        int pad_to, O* __restrict__ out) {
   norm_body<kNormMainWaves, N>(raw, items, n_items, blockIdx.x, pad_to, out);
+}
+
+// Long items, in segments of seg_frames(T) frames, chunks of 512 in registers.
+//
+// norm_segment leaves per (segment, slab) the sums S of (x - x0) and V of (x
+// - x0)^2, x0 the item's first value of the feature.  V comes from squared
+// deviations from the chunk's own f32 mean, moved to x0 in f64, so it carries
+// no f32 cancellation; it is exactly 0 where all values equal x0.
+// norm_finish adds the item's segments in order, has the sum of squared
+// deviations from the f32 mean m as V - 2 (m - x0) S + T (m - x0)^2 (f64: the
+// terms exceed it at most about T-fold), and writes its segment.
+//
+// What bounds it: memory.  One workgroup per (item, slab) streaming the item
+// three times left 24 clips of 20-90 s on 192 workgroups (79 us); segments
+// read it twice, the second time mostly from the Infinity Cache, and fill the
+// machine: 15 us for the sums (67 MB, 4.5 TB/s) and 26 us for the rest (67 MB
+// in, 67 MB out, 5.2 TB/s).  Shorter items stay whole: held in registers they
+// are read once, and 256 clips of 1-20 s take 49 us.
+constexpr int kSegRounds = kSegFrames / (kTile * kNormMainWaves);
+
+__device__ __forceinline__ void norm_segment(const float* __restrict__ raw, const Item* __restrict__ items,
+                                             const int32_t* __restrict__ seg_item, int work,
+                                             double2* __restrict__ parts) {
+  constexpr int W = kNormMainWaves;
+  constexpr int kSpan = NormShape<W>::kSpan;
+  __shared__ double red[W * kSlabF];
+  const int seg = work / kSlabs, slab = work % kSlabs;
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;
+  const Item it = items[seg_item[seg]];
+  const int sf = seg_frames(it.T), t0 = sf * (seg - it.seg0);
+  const int t1 = t0 + sf < it.T ? t0 + sf : it.T;
+  const float x0 = raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)] * kLn2;
+  double S = 0.0, V = 0.0;
+  for (int t = t0; t < t1; t += kSegFrames) {
+    const int n = t1 - t < kSegFrames ? t1 - t : kSegFrames;
+    const Rounds<W> rd(raw, it, slab, lane, w, t / kQuad);
+    const __amdgpu_buffer_rsrc_t rsrc = rd.buffer();
+    float4 v[kSegRounds];
+#pragma unroll
+    for (int j = 0; j < kSegRounds; ++j)
+      v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
+    double s = 0.0, sq = 0.0;
+#pragma unroll
+    for (int j = 0; j < kSegRounds; ++j) {
+      v[j] = ln2_scale(v[j]);
+      add_dev(s, v[j], x0, Rounds<W>::full(j, n), rd.left - kSpan * j);
+    }
+    s = slab_sum<W>(s, red, lane, w);
+    const float m = row_mean(x0, s, n);
+#pragma unroll
+    for (int j = 0; j < kSegRounds; ++j) add_sq(sq, v[j], m, Rounds<W>::full(j, n), rd.left - kSpan * j);
+    sq = slab_sum<W>(sq, red, lane, w);
+    const double d = (double)m - (double)x0, r = s - n * d;  // r: sum of (x - m)
+    S += s;
+    V += sq + 2.0 * d * r + n * (d * d);
+  }
+  if (w == 0 && lane < kSlabF) parts[(size_t)work * kSlabF + lane] = make_double2(S, V);
+}
+
+template <typename O>
+__device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const Item* __restrict__ items,
+                                            const int32_t* __restrict__ seg_item, int work,
+                                            const double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
+  constexpr int W = kNormMainWaves;
+  using NS = NormShape<W>;
+  __shared__ double red[W * kSlabF];
+  __shared__ float st[3 * kSlabF];
+  __shared__ __align__(16) float tb[2][kSlabF * NS::kTStride];
+  const int seg = work / kSlabs, slab = work % kSlabs;
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;
+  const Item it = items[seg_item[seg]];
+  const int T = it.T;
+  const int sf = seg_frames(T), n_segs = (T - 1) / sf + 1, t0 = sf * (seg - it.seg0);
+  const int t1 = t0 + sf < T ? t0 + sf : T;
+  const int rs = pad_to > 0 ? pad_to : T;
+  O* ob = out + it.dst_off + (size_t)(kSlabF * slab) * rs;
+  if (pad_to > 0 && t1 == T) zero_tail<W>(ob, T, rs, lane, w);
+  const float x0 = raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)] * kLn2;
+  float4 v[kSegRounds];
+  auto load = [&](int t) {
+    const Rounds<W> rd(raw, it, slab, lane, w, t / kQuad);
+    const __amdgpu_buffer_rsrc_t rsrc = rd.buffer();
+#pragma unroll
+    for (int j = 0; j < kSegRounds; ++j)
+      v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
+  };
+  load(t0);
+  // Segment k of the item: wave k % 4, lanes 16 (k / 4 % 4) ..
+  double S = 0.0, V = 0.0;
+  for (int k = w + W * (lane >> 4); k < n_segs; k += 4 * W) {
+    const double2 p = parts[((size_t)(it.seg0 + k) * kSlabs + slab) * kSlabF + (lane & 15)];
+    S += p.x;
+    V += p.y;
+  }
+  S = slab_sum<W>(S, red, lane, w);
+  V = slab_sum<W>(V, red, lane, w);
+  const double d = (double)row_mean(x0, S, T) - (double)x0;
+  publish_stats(S, fmax(V - 2.0 * d * S + T * (d * d), 0.0), V == 0.0, x0, T, lane, w, st);
+  for (int t = t0; t < t1; t += kSegFrames) {
+    if (t > t0) load(t);
+#pragma unroll
+    for (int ch = 0; ch < kSegRounds / 4; ++ch) {
+#pragma unroll
+      for (int jr = 0; jr < 4; ++jr)
+        *reinterpret_cast<float4*>(tb[ch % 2] + (lane & 15) * NS::kTStride + NS::kSpan * jr + 16 * w +
+                                   kQuad * (lane >> 4)) = ln2_scale(v[4 * ch + jr]);
+      __syncthreads();
+      store_chunk<W>(tb[ch % 2], st, t + NS::kChunk * ch, t1, rs, lane, w, ob);
+    }
+  }
+}
+
+// Workgroups [0, 8 n_segs): the long items' segments; the rest normalise the
+// other items.
+template <int N, typename O>
+__global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_long_kernel(
+    const float* __restrict__ raw, const Item* __restrict__ items, int n_items, int n_segs,
+    const int32_t* __restrict__ seg_item, double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
+  const int b = blockIdx.x;
+  if (b < kSlabs * n_segs) norm_segment(raw, items, seg_item, b, parts);
+  else norm_body<kNormMainWaves, N>(raw, items, n_items, b - kSlabs * n_segs, pad_to, out);
+}
+
+template <typename O>
+__global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_finish_kernel(
+    const float* __restrict__ raw, const Item* __restrict__ items, const int32_t* __restrict__ seg_item,
+    const double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
+  norm_finish(raw, items, seg_item, blockIdx.x, parts, pad_to, out);
 }
 
 // Calls of few items (a clip, a small batch) leave most CUs idle with 4-wave
@@ -977,12 +1063,24 @@ hipError_t launch_logmel(const void* samples, int pcm, float pcm_scale, const It
 }
 
 template <typename O>
-hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int max_T, int pad_to, O* out,
-                         hipStream_t stream) {
+hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int max_T, int pad_to, O* out, int n_segs,
+                         const int32_t* seg_item, double2* parts, hipStream_t stream) {
   using S = NormShape<kNormMainWaves>;
   using SW = NormShape<kNormWideWaves>;
   const unsigned blocks = (unsigned)((int64_t)n_items * kSlabs);
-  if (n_items <= kNormWideMaxItems && max_T <= SW::kSpan * 16) {
+  if (n_segs > 0) {
+    // Long items among them: their segments' sums beside the other items,
+    // then the segments themselves.
+    const unsigned seg_blocks = (unsigned)((int64_t)n_segs * kSlabs);
+    sfe_norm_long_kernel<kNormRegFrames / S::kSpan, O><<<dim3(seg_blocks + blocks), dim3(S::kThreads), 0, stream>>>(
+        raw, items, n_items, n_segs, seg_item, parts, pad_to, out);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    sfe_norm_finish_kernel<O><<<dim3(seg_blocks), dim3(S::kThreads), 0, stream>>>(raw, items, seg_item, parts, pad_to,
+                                                                                 out);
+    return hipGetLastError();
+  }
+  if (n_items <= kNormWideMaxItems) {
     const dim3 grid(blocks), block(SW::kThreads);
     if (max_T <= SW::kSpan * 8) sfe_norm_wide_kernel<8, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
     else sfe_norm_wide_kernel<16, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
@@ -990,7 +1088,7 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
   }
   const dim3 grid(blocks), block(S::kThreads);
   // Registers per lane sized to the longest item (N float4s hold kSpan N
-  // frames); longer ones take the streaming path.
+  // frames).
   if (max_T <= S::kSpan * 8) sfe_norm_kernel<8, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
   else if (max_T <= S::kSpan * 16) sfe_norm_kernel<16, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
   else if (max_T <= S::kSpan * 24) sfe_norm_kernel<24, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
@@ -999,10 +1097,12 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
 }
 
 hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int pad_to, void* out,
-                       bool out_bf16, hipStream_t stream) {
+                       bool out_bf16, int n_segs, const int32_t* seg_item, void* parts, hipStream_t stream) {
   if (n_items <= 0) return hipSuccess;
-  if (out_bf16) return launch_norm_t(raw, items, n_items, max_T, pad_to, static_cast<uint16_t*>(out), stream);
-  return launch_norm_t(raw, items, n_items, max_T, pad_to, static_cast<float*>(out), stream);
+  double2* p = static_cast<double2*>(parts);
+  if (out_bf16)
+    return launch_norm_t(raw, items, n_items, max_T, pad_to, static_cast<uint16_t*>(out), n_segs, seg_item, p, stream);
+  return launch_norm_t(raw, items, n_items, max_T, pad_to, static_cast<float*>(out), n_segs, seg_item, p, stream);
 }
 
 }  // namespace sfe

@@ -7,7 +7,8 @@
 // is looked up once per device with hipGetSymbolAddress (with that device
 // current) and only that address is passed to kernels and copies.
 //
-// Layout: [item table: kNoAllocItemBytes][raw log-mel: kNoAllocRawBytes].
+// Layout: [item table: kNoAllocItemBytes][raw log-mel: kNoAllocRawBytes]
+// [partial sums of long items: kNoAllocPartBytes].
 // Every call on one GPU shares the array: calls are serialised on the host
 // by a per-device lock and ordered on the device by a per-device event, so
 // calls from several contexts, threads or streams of one process do not
@@ -21,7 +22,7 @@
 namespace sfe {
 
 static_assert(kNoAllocItemBytes % 256 == 0, "raw region stays 256-byte aligned");
-static __device__ __align__(256) unsigned char scratch[kNoAllocItemBytes + kNoAllocRawBytes];
+static __device__ __align__(256) unsigned char scratch[kNoAllocItemBytes + kNoAllocRawBytes + kNoAllocPartBytes];
 
 namespace {
 

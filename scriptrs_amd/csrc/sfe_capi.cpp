@@ -162,6 +162,81 @@ struct PinBuf {
   }
 };
 
+// Pinned staging of the calls' tables, read by their uploads: a buffer of two
+// halves.  take() hands out consecutive pieces of the current half; when it is
+// full, an event on the caller's stream marks the end of its uploads, and the
+// other half is free once its own event (a half ago) has passed.  An event
+// after every upload, waited for by the next call, cost each call a marker
+// between its upload and its first kernel (5.6 us on the device) and held the
+// host to one call ahead.  The calls of a context are ordered after each
+// other, also across streams, so the event covers the whole half.
+struct PinRing {
+  char* ptr = nullptr;
+  size_t half = 0, at = 0;  // at: bytes used of the current half
+  int cur = 0;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  bool pending[2] = {false, false};
+  hipError_t wait(int h) {
+    if (!pending[h]) return hipSuccess;
+    pending[h] = false;
+    return hipEventSynchronize(ev[h]);
+  }
+  // Room for pieces of up to `bytes`.  Growing waits for the device: uploads
+  // from the old buffer may be queued on any stream.
+  hipError_t reserve(size_t bytes) {
+    hipError_t e;
+    for (int h = 0; h < 2; ++h)
+      if (!ev[h] && (e = hipEventCreateWithFlags(&ev[h], hipEventDisableTiming)) != hipSuccess) {
+        ev[h] = nullptr;
+        return e;
+      }
+    const size_t want = (std::max(bytes, (size_t)4096) + 255) / 256 * 256;
+    if (want <= half) return hipSuccess;
+    if (ptr) {
+      if ((e = hipDeviceSynchronize()) != hipSuccess) return e;
+      (void)hipHostFree(ptr);
+      ptr = nullptr;
+      half = 0;
+    }
+    void* p = nullptr;
+    e = hipHostMalloc(&p, 2 * want, hipHostMallocDefault);
+    g_allocations.fetch_add(1);
+    if (e != hipSuccess) return e;
+    ptr = static_cast<char*>(p);
+    half = want;
+    at = 0;
+    cur = 0;
+    pending[0] = pending[1] = false;
+    return hipSuccess;
+  }
+  // The next `bytes` (256-byte aligned), for an upload on `stream`, on which
+  // the context's earlier calls are ordered.
+  hipError_t take(size_t bytes, hipStream_t stream, char** out) {
+    hipError_t e = reserve(bytes);
+    if (e != hipSuccess) return e;
+    const size_t n = (bytes + 255) / 256 * 256;
+    if (at + n > half) {
+      if ((e = hipEventRecord(ev[cur], stream)) != hipSuccess) return e;
+      pending[cur] = true;
+      cur ^= 1;
+      at = 0;
+      if ((e = wait(cur)) != hipSuccess) return e;
+    }
+    *out = ptr + (size_t)cur * half + at;
+    at += n;
+    return hipSuccess;
+  }
+  void release() {
+    if (ptr) (void)hipHostFree(ptr);
+    for (hipEvent_t& v : ev) {
+      if (v) (void)hipEventDestroy(v);
+      v = nullptr;
+    }
+    ptr = nullptr;
+    half = 0;
+  }
+};
+
 bool shape_supported(const sfe_config* c, std::string* why) {
   if (c->n_fft != sfe::kNfft || c->win_length != sfe::kWin || c->hop_length != sfe::kHop ||
       c->feature_size != sfe::kMel) {
@@ -198,7 +273,7 @@ struct sfe_ctx {
   bool last_marked = false;   // ev_last marks the end of the previous call
   bool multi_stream = false;  // calls have come on more than one stream
   hipStream_t last_stream = nullptr;  // the stream the previous call's device work ran on
-  PinBuf h_meta;
+  PinRing h_meta;
   DevBuf scratch;   // raw log-mel in 16-frame tiles, f32 (the normalisation kernel's input)
   DevBuf parts;     // partial sums of long items' segments (sfe::launch_norm)
   DevBuf io_in;     // sfe_extract staging (audio)
@@ -401,27 +476,26 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
   // earlier work still in flight is unaffected.
   const bool same = ctx->meta.ptr && ctx->meta_items.size() == table.size() &&
                     memcmp(ctx->meta_items.data(), table.data(), tbytes) == 0;
+  SFE_HIP(ctx->scratch.reserve((size_t)total_tiles * sfe::kRawTile * sizeof(float)));
+  SFE_HIP(ctx->parts.reserve((size_t)ctx->plan_segs * sfe::kSegPartBytes));
   if (!same) {
     ctx->meta_items.clear();
-    SFE_HIP(ctx->h_meta.reserve(mbytes));
-    SFE_HIP(ctx->meta.reserve(mbytes));
-    memcpy(ctx->h_meta.ptr, table.data(), tbytes);
+    SFE_HIP(ctx->meta.reserve(mbytes + 16));
+    char* stage = nullptr;
+    SFE_HIP(ctx->h_meta.take(mbytes, stream, &stage));
+    memcpy(stage, table.data(), tbytes);
     if (wt.entries)
       sfe::logmel_wave_items(table.data(), (int)n_lm, wt.u0, wt.n_units, wt.grid,
-                             reinterpret_cast<int32_t*>(static_cast<char*>(ctx->h_meta.ptr) + tbytes));
+                             reinterpret_cast<int32_t*>(stage + tbytes));
     if (ctx->plan_segs > 0)
       sfe::norm_segments(ctx->plan_table.data() + n_lm, (int)items.size(),
-                         reinterpret_cast<int32_t*>(static_cast<char*>(ctx->h_meta.ptr) + sbytes));
-    SFE_HIP(hipMemcpyAsync(ctx->meta.ptr, ctx->h_meta.ptr, mbytes, hipMemcpyHostToDevice, stream));
-    SFE_HIP(hipEventRecord(ctx->h_meta.ev, stream));
-    ctx->h_meta.pending = true;
+                         reinterpret_cast<int32_t*>(stage + sbytes));
+    SFE_HIP(sfe::launch_upload(stage, ctx->meta.ptr, mbytes, stream));
     ctx->meta_items = table;
   }
   const Item* d_table = static_cast<const Item*>(ctx->meta.ptr);
   const int32_t* d_wave =
       wt.entries ? reinterpret_cast<const int32_t*>(static_cast<const char*>(ctx->meta.ptr) + tbytes) : nullptr;
-  SFE_HIP(ctx->scratch.reserve((size_t)total_tiles * sfe::kRawTile * sizeof(float)));
-  SFE_HIP(ctx->parts.reserve((size_t)ctx->plan_segs * sfe::kSegPartBytes));
   float* raw = static_cast<float*>(ctx->scratch.ptr);
   const Segments segs{(int)ctx->plan_segs,
                       reinterpret_cast<const int32_t*>(static_cast<const char*>(ctx->meta.ptr) + sbytes),
@@ -847,7 +921,7 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
       SFE_HIP(sfe::noalloc_scratch(ctx->device, &na));
       ctx->noalloc = static_cast<unsigned char*>(na);
     }
-    if (ctx->h_meta.cap <
+    if (ctx->h_meta.half <
             entries * sizeof(Item) + (sfe::kMaxLogmelWaves + sfe::kNoAllocMaxSegs) * sizeof(int32_t) ||
         ctx->na_in.capacity() < (size_t)n)
       return fail(SFE_HIP_ERROR, "context has no reserved planner buffers");
@@ -862,9 +936,12 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
       own_tiles += sfe::tiles_for(it.T);
       frame_offsets[i + 1] = fo;
     }
-    // The pinned table is free once its previous upload has finished.
-    SFE_HIP(ctx->h_meta.wait());
-    Item* table = static_cast<Item*>(ctx->h_meta.ptr);
+    SFE_HIP(order_after_last(ctx, s));
+    SFE_HIP(sfe::noalloc_order(ctx->device, s));
+    char* stage = nullptr;
+    SFE_HIP(ctx->h_meta.take(entries * sizeof(Item) + (sfe::kMaxLogmelWaves + sfe::kNoAllocMaxSegs) * sizeof(int32_t),
+                             s, &stage));
+    Item* table = reinterpret_cast<Item*>(stage);
     size_t n_lm = 0;
     bool share = ctx->share;
     tiles = sfe::plan_table(ctx->na_in.data(), n, share, &ctx->na_ws, table, &n_lm);
@@ -872,8 +949,6 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
     sfe::order_norm(table + n_lm, n);
     const int64_t n_segs = sfe::norm_segments(table + n_lm, n, nullptr);
     if (n_segs > sfe::kNoAllocMaxSegs) return fail(SFE_HIP_ERROR, "segments outgrow the static scratch");
-    SFE_HIP(order_after_last(ctx, s));
-    SFE_HIP(sfe::noalloc_order(ctx->device, s));
     Item* d_table = reinterpret_cast<Item*>(ctx->noalloc);
     float* raw = reinterpret_cast<float*>(ctx->noalloc + sfe::kNoAllocItemBytes);
     // the table, then the log-mel launch's first-item table and the long
@@ -891,9 +966,7 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
       sfe::norm_segments(table + n_lm, n, reinterpret_cast<int32_t*>(reinterpret_cast<char*>(table) + sbytes));
     const Segments segs{(int)n_segs, reinterpret_cast<const int32_t*>(ctx->noalloc + sbytes),
                         ctx->noalloc + sfe::kNoAllocItemBytes + sfe::kNoAllocRawBytes};
-    SFE_HIP(hipMemcpyAsync(d_table, table, sbytes + (size_t)n_segs * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    SFE_HIP(hipEventRecord(ctx->h_meta.ev, s));
-    ctx->h_meta.pending = true;
+    SFE_HIP(sfe::launch_upload(table, d_table, sbytes + (size_t)n_segs * sizeof(int32_t), s));
     rc = launch_pair(ctx, f32_source(recording), table, d_table, (int)n_lm, table + n_lm, d_table + n_lm, n, segs, raw, out,
                      out_dtype, 0, s, kBoth, false, d_wave);
     if (rc) return rc;
@@ -1130,18 +1203,17 @@ int sfe_extract_chunks_streamed_pcm(sfe_ctx* ctx, const void* host_recording, in
     const size_t tbytes = table.size() * sizeof(Item);
     const size_t mbytes = tbytes + (size_t)total_segs * sizeof(int32_t);
     ctx->meta_items.clear();  // the table uploaded below is re-based per window group
-    SFE_HIP(ctx->h_meta.reserve(mbytes));
-    SFE_HIP(ctx->meta.reserve(mbytes));
+    SFE_HIP(ctx->meta.reserve(mbytes + 16));
+    char* stage = nullptr;
+    SFE_HIP(ctx->h_meta.take(mbytes, sc, &stage));
     SFE_HIP(ctx->scratch.reserve((size_t)tiles * sfe::kRawTile * sizeof(float)));
     SFE_HIP(ctx->parts.reserve((size_t)max_segs * sfe::kSegPartBytes));
     float* raw = static_cast<float*>(ctx->scratch.ptr);
-    memcpy(ctx->h_meta.ptr, table.data(), tbytes);
-    int32_t* seg_list = reinterpret_cast<int32_t*>(static_cast<char*>(ctx->h_meta.ptr) + tbytes);
+    memcpy(stage, table.data(), tbytes);
+    int32_t* seg_list = reinterpret_cast<int32_t*>(stage + tbytes);
     for (const NormGroup& g : norm_groups)
       if (g.n_segs > 0) sfe::norm_segments(nm_tab.data() + g.first, g.end - g.first, seg_list + g.seg0);
-    SFE_HIP(hipMemcpyAsync(ctx->meta.ptr, ctx->h_meta.ptr, mbytes, hipMemcpyHostToDevice, sc));
-    SFE_HIP(hipEventRecord(ctx->h_meta.ev, sc));
-    ctx->h_meta.pending = true;
+    SFE_HIP(sfe::launch_upload(stage, ctx->meta.ptr, mbytes, sc));
     const Item* d_items = static_cast<const Item*>(ctx->meta.ptr);
     Source rsrc = src;
     rsrc.ptr = ring;

@@ -219,6 +219,9 @@ int64_t units_for(int64_t T);  // quads of an item: ceil(T / 4)
 constexpr int kPcmF32 = 0;
 constexpr int kPcmI16 = 1;
 constexpr int kPcmI32 = 2;
+// Copies bytes (rounded up to 16; both sides 16-byte aligned and with room for
+// that) from pinned host memory to the device with a kernel on `stream`.
+hipError_t launch_upload(const void* src, void* dst, size_t bytes, hipStream_t stream);
 // Units [unit0, unit0 + n_units) in the numbering of items[].unit_off.
 // Timestamp buffer of measurement builds (-DSFE_TIMESTAMPS, sfe_kernels.hip);
 // stamps_built() is false and set_stamp_buffer fails in the product build.

@@ -105,6 +105,9 @@ def _ip(a: np.ndarray):
 def _stream_handle(stream) -> ctypes.c_void_p:
     if stream is None:
         import torch
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:  # torch.cuda.current_stream().cuda_stream without its Stream object
+            return ctypes.c_void_p(raw(torch.cuda.current_device()))
         stream = torch.cuda.current_stream()
     return ctypes.c_void_p(int(getattr(stream, "cuda_stream", stream)))
 
@@ -210,14 +213,16 @@ class ParakeetFeatureExtractor:
         n = off.size - 1
         if n <= 0:
             raise InvalidModelOutput("need at least one clip")
-        if off[0] < 0 or np.any(np.diff(off) < 0):
+        lens = off[1:] - off[:-1]
+        shortest = lens.min()
+        if off[0] < 0 or shortest < 0:
             raise InvalidModelOutput("offsets must be non-negative and non-decreasing")
         if off[-1] > samples.numel():
             raise InvalidModelOutput(f"offsets run to {int(off[-1])}, past the {samples.numel()} samples")
-        if np.any(np.diff(off) == 0):
+        if shortest == 0:
             raise EmptyAudio()
         fo = np.zeros(n + 1, np.int64)
-        fo[1:] = np.cumsum(np.diff(off) // self.config.hop_length + 1)
+        np.cumsum(lens // self.config.hop_length + 1, out=fo[1:])
         if out is None:
             out = torch.empty(int(fo[-1]) * self.config.feature_size, dtype=_torch_dtype(dtype), device=samples.device)
         _check_out(out, dtype, int(fo[-1]) * self.config.feature_size)

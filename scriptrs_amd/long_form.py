@@ -20,7 +20,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import SfeChunk, SfeOverlapConfig
-from .frontend import EmptyAudio, InvalidModelOutput, ParakeetFeatureExtractor, TranscriptionConfig
+from .frontend import EmptyAudio, InvalidModelOutput, ParakeetFeatureExtractor, TaskTable, TranscriptionConfig
 
 
 @dataclass(frozen=True)
@@ -48,21 +48,26 @@ class OverlapChunkConfig:
     def _c(self) -> SfeOverlapConfig:
         return SfeOverlapConfig(self.overlap_seconds, self.context_samples, self.max_model_samples)
 
-    def tasks(self, audio_len: int) -> list[ChunkTask]:
-        """``plan`` over [0, audio_len) mapped through ``push_overlap_task``."""
+    def _table(self, audio_len: int) -> np.ndarray:
+        """``tasks`` as an int64 array in the C ABI's layout, [n, 4]."""
         L = _lib.lib()
         c = self._c()
         n = ctypes.c_int32(0)
         rc = L.sfe_plan_fast(ctypes.byref(c), int(audio_len), None, 0, ctypes.byref(n))
         if n.value == 0:
-            return []
+            return np.zeros((0, 4), np.int64)
         if rc not in (_lib.SFE_OK, _lib.SFE_INVALID_ARG):
             raise InvalidModelOutput(_lib.last_error())
-        arr = (SfeChunk * n.value)()
-        rc = L.sfe_plan_fast(ctypes.byref(c), int(audio_len), arr, n.value, ctypes.byref(n))
+        a = np.empty((n.value, 4), np.int64)
+        rc = L.sfe_plan_fast(ctypes.byref(c), int(audio_len), a.ctypes.data_as(ctypes.POINTER(SfeChunk)), n.value,
+                             ctypes.byref(n))
         if rc != _lib.SFE_OK:
             raise InvalidModelOutput(_lib.last_error())
-        return [ChunkTask(t.audio_start, t.audio_end, t.global_sample_offset, t.context_samples) for t in arr]
+        return a
+
+    def tasks(self, audio_len: int) -> list[ChunkTask]:
+        """``plan`` over [0, audio_len) mapped through ``push_overlap_task``."""
+        return [ChunkTask(*t) for t in self._table(audio_len).tolist()]
 
     def plan(self, rng: SampleRange) -> list[SampleRange]:
         """``OverlapChunkConfig::plan`` (src/long_form/planner.rs:124-137) over ``rng``."""
@@ -117,8 +122,11 @@ def featurize_long_form(extractor: ParakeetFeatureExtractor, recording, config: 
     if n == 0:
         raise EmptyAudio()
     if n <= cfg.transcription.max_audio_samples:
-        tasks = [ChunkTask(0, n, 0, 0)]
+        table = np.array([[0, n, 0, 0]], np.int64)
     else:
-        tasks = build_fast_execution_plan(n, cfg)
-    out, fo = extractor.extract_chunks(recording, tasks, dtype=dtype, stream=stream)
+        table = cfg.overlap._table(n)
+    # (the call is enqueued first: the GPU works while the task list is made)
+    out, fo = extractor.extract_chunks(recording, TaskTable(table, extractor.config.hop_length), dtype=dtype,
+                                       stream=stream)
+    tasks = [ChunkTask(*t) for t in table.tolist()]
     return LongFormFeatures(tasks, out, fo, cfg.transcription.feature_size)

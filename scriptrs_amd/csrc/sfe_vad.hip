@@ -15,7 +15,7 @@
 // tensors back to back), decoding integer PCM on the fly.  It moves
 // 4 B/sample in (f32; 2 for 16-bit PCM) and 4.5 B/sample out, and is bound
 // by HBM bandwidth: no arithmetic beyond the decode.  The 64-sample context
-// re-read hits L2 (the neighbouring window is read by the same workgroup).
+// re-read hits L2 (the neighbouring window is mostly the same workgroup's).
 
 #include <hip/hip_runtime.h>
 
@@ -28,12 +28,22 @@ namespace sfe {
 namespace {
 
 constexpr int kVadRowVec = kVadRow / 4;   // 144 float4 per model input
-constexpr int kVadThreads = 256;
-constexpr int kVadRowsPerBlock = 16;
-constexpr int kVadVecPerThread = kVadRowsPerBlock * kVadRowVec / kVadThreads;  // 9
-static_assert(kVadRowsPerBlock * kVadRowVec % kVadThreads == 0, "whole float4s per thread");
+// One float4 of output per thread: 576 threads, 9 whole waves, write 4 rows.
+// What bounds it: memory, and how evenly the workgroups keep it busy.  With 9
+// float4s per thread (16 rows of 256 threads) the 1 h recording took 90 us (490
+// MB, 5.4 TB/s; 71 us for 16-bit PCM), with 3 (192 threads) 84, with one 80
+// and 61; 288 threads (4.5 waves) 78 and 67.
+constexpr int kVadRowsPerBlock = 4;
+constexpr int kVadThreads = kVadRowsPerBlock * kVadRowVec;  // 576
+static_assert(kVadThreads % 64 == 0, "whole waves");
 static_assert(kVadCtx % 4 == 0 && kVadWin % 4 == 0, "rows start on float4 boundaries of the recording");
 
+// Recordings whose samples and rows together exceed the 256 MB Infinity Cache
+// are read past the caches where a sample is 4 bytes: 1 h 75 us against 80
+// with plain loads, 2 h 155 against 162.  Smaller ones, whose samples may
+// still be cached, are not (20 min 26 us against 23, 1 min 3.4 against 2.7),
+// and 16-bit PCM is not at any size measured (1 h 64 us against 61).
+constexpr int64_t kVadStreamBytes = (int64_t)256 << 20;
 
 template <typename S>
 __device__ __forceinline__ float vad_sample(const S* x, int64_t len, int64_t i, const Decode& d) {
@@ -41,42 +51,41 @@ __device__ __forceinline__ float vad_sample(const S* x, int64_t len, int64_t i, 
   return Pcm<S>::dec(x[i < len ? i : len - 1], d);
 }
 
-// One workgroup writes kVadRowsPerBlock model inputs; thread t handles the
-// float4s t, t + 256, ... of the block's rows, so a wave's loads and stores
-// are contiguous except across a row boundary.  All loads are issued before
-// the first store.
-template <typename S>
+// One workgroup writes kVadRowsPerBlock model inputs, thread t float4 t of
+// them, so a wave's loads and stores are contiguous except across a row
+// boundary.  STREAM: nontemporal loads.
+template <typename S, bool STREAM>
 __global__ __launch_bounds__(kVadThreads) void sfe_vad_frames_kernel(const S* __restrict__ x, int64_t len,
                                                                      int64_t n_windows, Decode dc,
                                                                      float* __restrict__ out) {
-  const int64_t row0 = (int64_t)blockIdx.x * kVadRowsPerBlock;
-  float4 v[kVadVecPerThread];
-  int64_t dst[kVadVecPerThread];
-#pragma unroll
-  for (int k = 0; k < kVadVecPerThread; ++k) {
-    const int e = (int)threadIdx.x + kVadThreads * k;  // float4 index in the block
-    const int r = e / kVadRowVec;
-    const int p = 4 * (e - r * kVadRowVec);
-    const int64_t w = row0 + r;
-    const int64_t i = w * kVadWin - kVadCtx + p;
-    dst[k] = w < n_windows ? w * kVadRow + p : -1;
-    if (i >= 0 && i + 4 <= len) {
-      v[k] = Pcm<S>::dec4(Pcm<S>::load4(x + i), dc);
-    } else {
-      v[k] = make_float4(vad_sample(x, len, i, dc), vad_sample(x, len, i + 1, dc), vad_sample(x, len, i + 2, dc),
-                         vad_sample(x, len, i + 3, dc));
-    }
+  const int r = (int)threadIdx.x / kVadRowVec;
+  const int p = 4 * ((int)threadIdx.x - r * kVadRowVec);
+  const int64_t w = (int64_t)blockIdx.x * kVadRowsPerBlock + r;
+  if (w >= n_windows) return;
+  const int64_t i = w * kVadWin - kVadCtx + p;
+  float4 v;
+  if (i >= 0 && i + 4 <= len) {
+    typedef typename Pcm<S>::V4 V4;
+    const V4* q = reinterpret_cast<const V4*>(x + i);
+    v = Pcm<S>::dec4(STREAM ? __builtin_nontemporal_load(q) : *q, dc);
+  } else {
+    v = make_float4(vad_sample(x, len, i, dc), vad_sample(x, len, i + 1, dc), vad_sample(x, len, i + 2, dc),
+                    vad_sample(x, len, i + 3, dc));
   }
-  // Nontemporal stores: the output is not read again by this kernel, and
-  // streaming it past the caches measured 73 us against 96 us for plain
-  // stores on the 1 h recording.
+  // Nontemporal stores: the output is not read again by this kernel (1 h
+  // recording 78 us against 82 with plain stores).
   typedef float F4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-  for (int k = 0; k < kVadVecPerThread; ++k)
-    if (dst[k] >= 0) {
-      const F4 t = {v[k].x, v[k].y, v[k].z, v[k].w};
-      __builtin_nontemporal_store(t, reinterpret_cast<F4*>(out + dst[k]));
-    }
+  __builtin_nontemporal_store(F4{v.x, v.y, v.z, v.w}, reinterpret_cast<F4*>(out + w * kVadRow + p));
+}
+
+template <typename S>
+void launch_vad(const void* samples, int64_t len, int64_t n, const Decode& dc, float* out, hipStream_t stream) {
+  const dim3 g((unsigned)((n + kVadRowsPerBlock - 1) / kVadRowsPerBlock)), b(kVadThreads);
+  const S* x = static_cast<const S*>(samples);
+  if (sizeof(S) == 4 && 4 * (len + kVadRow * n) > kVadStreamBytes)
+    sfe_vad_frames_kernel<S, true><<<g, b, 0, stream>>>(x, len, n, dc, out);
+  else
+    sfe_vad_frames_kernel<S, false><<<g, b, 0, stream>>>(x, len, n, dc, out);
 }
 
 }  // namespace
@@ -87,14 +96,10 @@ hipError_t launch_vad_frames(const void* samples, int pcm, float pcm_scale, int6
                              hipStream_t stream) {
   const int64_t n = vad_num_windows(len);
   if (n == 0) return hipSuccess;
-  const dim3 g((unsigned)((n + kVadRowsPerBlock - 1) / kVadRowsPerBlock)), b(kVadThreads);
   const Decode dc{pcm_scale, 1.0f / pcm_scale, 1.0 / (double)pcm_scale};
-  if (pcm == kPcmI16)
-    sfe_vad_frames_kernel<int16_t><<<g, b, 0, stream>>>(static_cast<const int16_t*>(samples), len, n, dc, out);
-  else if (pcm == kPcmI32)
-    sfe_vad_frames_kernel<int32_t><<<g, b, 0, stream>>>(static_cast<const int32_t*>(samples), len, n, dc, out);
-  else
-    sfe_vad_frames_kernel<float><<<g, b, 0, stream>>>(static_cast<const float*>(samples), len, n, dc, out);
+  if (pcm == kPcmI16) launch_vad<int16_t>(samples, len, n, dc, out, stream);
+  else if (pcm == kPcmI32) launch_vad<int32_t>(samples, len, n, dc, out, stream);
+  else launch_vad<float>(samples, len, n, dc, out, stream);
   return hipGetLastError();
 }
 

@@ -280,12 +280,14 @@ hipError_t launch_logmel(const void* samples, int pcm, float pcm_scale, const It
 // Normalises raw (f32 log2 values in 16-frame tiles, see Item) per (item, feature)
 // and writes feature-major [128][T] per item to out (f32, must not alias
 // raw) or bf16 (uint16_t*) when out_bf16 is set.  max_T: the longest item's
-// frame count (sizes the kernel's register budget).  pad_to > 0: rows of
+// frame count (sizes the kernel's register budget); sum_T: all items' frames;
+// cus: the device's compute units.  pad_to > 0: rows of
 // pad_to frames, zero past T (the encoder input layout).  n_segs, seg_item,
 // parts: the long items' segments (norm_segments over items), the device copy
 // of their entry indexes and n_segs * kSegPartBytes of scratch.
-hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int pad_to, void* out,
-                       bool out_bf16, int n_segs, const int32_t* seg_item, void* parts, hipStream_t stream);
+hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, int cus, int pad_to,
+                       void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
+                       hipStream_t stream);
 
 // Static scratch of the allocation-free entry point (sfe_noalloc.hip): an
 // item table of up to kNoAllocMaxItems items, then kNoAllocRawBytes of raw

@@ -168,6 +168,11 @@ __device__ __forceinline__ float4 ln2_scale(float4 v) {
   return make_float4(v.x * kLn2, v.y * kLn2, v.z * kLn2, v.w * kLn2);
 }
 
+__device__ __forceinline__ float ln2_scale(float v) {
+#pragma clang fp contract(off)
+  return v * kLn2;
+}
+
 // Raw log-mel is written in tiles of 16 frames: 8 slabs of 16 features, each
 // [4 quads][16 features][4 frames] (1 KB).  Lane L holds the quad's 4 frames
 // of filters L and 64 + L: two aligned 16-byte stores per lane, each store
@@ -562,18 +567,24 @@ struct NormShape {
   static_assert(4 * kLanesPerRow == kSpan, "a store instruction covers one round of a row");
 };
 
-// Workgroup sum of v over the lanes that hold the same feature (lane % 16
-// equal) and the waves; every lane gets its own feature's total.  red holds
-// 16 W doubles.
+// Workgroup sum over the lanes that hold the same feature (lane % 16 equal)
+// and the waves; every lane gets its own feature's total.  v[k] holds the
+// lane's sum over rounds j = k mod 8 / W: tile 4 j + w of a 4-wave workgroup is
+// tile 8 (j / 2) + w + 4 (j % 2) of an 8-wave one, so both add the same 8 sums
+// in the same order and the results do not depend on the form.
+constexpr int kSumParts = 8;
 template <int W>
-__device__ __forceinline__ double slab_sum(double v, double* red, int lane, int w) {
-  v += __shfl_xor(v, 16, 64);
-  v += __shfl_xor(v, 32, 64);
-  if (lane < kSlabF) red[w * kSlabF + lane] = v;
+__device__ __forceinline__ double slab_sum(double (&v)[kSumParts / W], double* red, int lane, int w) {
+#pragma unroll
+  for (int k = 0; k < kSumParts / W; ++k) {
+    v[k] += __shfl_xor(v[k], 16, 64);
+    v[k] += __shfl_xor(v[k], 32, 64);
+    if (lane < kSlabF) red[(w + W * k) * kSlabF + lane] = v[k];
+  }
   __syncthreads();
   double t = 0.0;
 #pragma unroll
-  for (int u = 0; u < W; ++u) t += red[u * kSlabF + lane % kSlabF];
+  for (int u = 0; u < kSumParts; ++u) t += red[u * kSlabF + lane % kSlabF];
   __syncthreads();  // red is reused by the next reduction
   return t;
 }
@@ -746,7 +757,7 @@ __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const I
   using S = NormShape<W>;
   constexpr int kSpan = S::kSpan;
   constexpr int kChunk = S::kChunk;
-  __shared__ double red[W * kSlabF];
+  __shared__ double red[kSumParts * kSlabF];
   __shared__ float st[3 * kSlabF];
   // Two transpose buffers in the 4-wave form (chunk ch stages into tb[ch %
   // 2]: the next chunk's staging does not wait for this chunk's stores, one
@@ -772,14 +783,15 @@ __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const I
   if (pad_to > 0) zero_tail<W>(ob, T, rs, lane, w);
   // Frame 0 is always at out_off: below f_lo for an item that shares frames,
   // and an item with its own region has grid_off = out_off.
-  const float x0 = raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)] * kLn2;
+  const float x0 = ln2_scale(raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)]);
   // The chunk's columns of this lane's quads.
   auto stage = [&](float* t, int jr, const float4& v) {
     *reinterpret_cast<float4*>(t + (lane & 15) * S::kTStride + kSpan * jr + kQuad * rd.q) = v;
   };
   const int chunks = (T + kChunk - 1) / kChunk;
 
-  double s = 0.0, sq = 0.0;
+  constexpr int K = kSumParts / W;
+  double sp[K] = {}, qp[K] = {};
   float4 v[N];
   // Raw buffer loads from the uniform base, all issued before any is used
   // (a load under a per-lane branch would wait for itself).
@@ -790,16 +802,16 @@ __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const I
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     v[j] = ln2_scale(v[j]);
-    add_dev(s, v[j], x0, Rounds<W>::full(j, T), rd.left - kSpan * j);
+    add_dev(sp[j % K], v[j], x0, Rounds<W>::full(j, T), rd.left - kSpan * j);
   }
-  s = slab_sum<W>(s, red, lane, w);
+  const double s = slab_sum<W>(sp, red, lane, w);
 #ifdef SFE_TIMESTAMPS
   if (threadIdx.x == 0) SFE_STAMP(sn + 1, stamp_now());
 #endif
   const float m = row_mean(x0, s, T);
 #pragma unroll
-  for (int j = 0; j < N; ++j) add_sq(sq, v[j], m, Rounds<W>::full(j, T), rd.left - kSpan * j);
-  sq = slab_sum<W>(sq, red, lane, w);
+  for (int j = 0; j < N; ++j) add_sq(qp[j % K], v[j], m, Rounds<W>::full(j, T), rd.left - kSpan * j);
+  const double sq = slab_sum<W>(qp, red, lane, w);
   publish_stats(s, sq, sq == 0.0, x0, T, lane, w, st);
 #ifdef SFE_TIMESTAMPS
   if (threadIdx.x == 0) SFE_STAMP(sn + 2, stamp_now());
@@ -866,14 +878,14 @@ __device__ __forceinline__ void norm_segment(const float* __restrict__ raw, cons
                                              double2* __restrict__ parts) {
   constexpr int W = kNormMainWaves;
   constexpr int kSpan = NormShape<W>::kSpan;
-  __shared__ double red[W * kSlabF];
+  __shared__ double red[kSumParts * kSlabF];
   const int seg = work / kSlabs, slab = work % kSlabs;
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const Item it = items[seg_item[seg]];
   const int sf = seg_frames(it.T), t0 = sf * (seg - it.seg0);
   const int t1 = t0 + sf < it.T ? t0 + sf : it.T;
-  const float x0 = raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)] * kLn2;
+  const float x0 = ln2_scale(raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)]);
   double S = 0.0, V = 0.0;
   for (int t = t0; t < t1; t += kSegFrames) {
     const int n = t1 - t < kSegFrames ? t1 - t : kSegFrames;
@@ -883,17 +895,18 @@ __device__ __forceinline__ void norm_segment(const float* __restrict__ raw, cons
 #pragma unroll
     for (int j = 0; j < kSegRounds; ++j)
       v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
-    double s = 0.0, sq = 0.0;
+    constexpr int K = kSumParts / W;
+    double sp[K] = {}, qp[K] = {};
 #pragma unroll
     for (int j = 0; j < kSegRounds; ++j) {
       v[j] = ln2_scale(v[j]);
-      add_dev(s, v[j], x0, Rounds<W>::full(j, n), rd.left - kSpan * j);
+      add_dev(sp[j % K], v[j], x0, Rounds<W>::full(j, n), rd.left - kSpan * j);
     }
-    s = slab_sum<W>(s, red, lane, w);
+    const double s = slab_sum<W>(sp, red, lane, w);
     const float m = row_mean(x0, s, n);
 #pragma unroll
-    for (int j = 0; j < kSegRounds; ++j) add_sq(sq, v[j], m, Rounds<W>::full(j, n), rd.left - kSpan * j);
-    sq = slab_sum<W>(sq, red, lane, w);
+    for (int j = 0; j < kSegRounds; ++j) add_sq(qp[j % K], v[j], m, Rounds<W>::full(j, n), rd.left - kSpan * j);
+    const double sq = slab_sum<W>(qp, red, lane, w);
     const double d = (double)m - (double)x0, r = s - n * d;  // r: sum of (x - m)
     S += s;
     V += sq + 2.0 * d * r + n * (d * d);
@@ -907,7 +920,7 @@ __device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const
                                             const double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
   constexpr int W = kNormMainWaves;
   using NS = NormShape<W>;
-  __shared__ double red[W * kSlabF];
+  __shared__ double red[kSumParts * kSlabF];
   __shared__ float st[3 * kSlabF];
   __shared__ __align__(16) float tb[2][kSlabF * NS::kTStride];
   const int seg = work / kSlabs, slab = work % kSlabs;
@@ -920,7 +933,7 @@ __device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const
   const int rs = pad_to > 0 ? pad_to : T;
   O* ob = out + it.dst_off + (size_t)(kSlabF * slab) * rs;
   if (pad_to > 0 && t1 == T) zero_tail<W>(ob, T, rs, lane, w);
-  const float x0 = raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)] * kLn2;
+  const float x0 = ln2_scale(raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)]);
   float4 v[kSegRounds];
   auto load = [&](int t) {
     const Rounds<W> rd(raw, it, slab, lane, w, t / kQuad);
@@ -931,14 +944,14 @@ __device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const
   };
   load(t0);
   // Segment k of the item: wave k % 4, lanes 16 (k / 4 % 4) ..
-  double S = 0.0, V = 0.0;
+  double Sp[kSumParts / W] = {}, Vp[kSumParts / W] = {};
   for (int k = w + W * (lane >> 4); k < n_segs; k += 4 * W) {
     const double2 p = parts[((size_t)(it.seg0 + k) * kSlabs + slab) * kSlabF + (lane & 15)];
-    S += p.x;
-    V += p.y;
+    Sp[0] += p.x;
+    Vp[0] += p.y;
   }
-  S = slab_sum<W>(S, red, lane, w);
-  V = slab_sum<W>(V, red, lane, w);
+  const double S = slab_sum<W>(Sp, red, lane, w);
+  const double V = slab_sum<W>(Vp, red, lane, w);
   const double d = (double)row_mean(x0, S, T) - (double)x0;
   publish_stats(S, fmax(V - 2.0 * d * S + T * (d * d), 0.0), V == 0.0, x0, T, lane, w, st);
   for (int t = t0; t < t1; t += kSegFrames) {
@@ -973,12 +986,22 @@ __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_finish_kernel(
   norm_finish(raw, items, seg_item, blockIdx.x, parts, pad_to, out);
 }
 
-// Calls of few items (a clip, a small batch) leave most CUs idle with 4-wave
-// workgroups, and each workgroup's loads, reductions and stores run one
-// after another: 8-wave workgroups (128 frames per round, 33 KB of LDS for
-// the 512-frame transpose chunks) put twice the waves on each slab.
+// 8-wave workgroups (128 frames per round, 33 KB of LDS for the 512-frame
+// transpose chunks, half the registers per lane, 3 per CU) against 4-wave
+// ones (4 per CU in the 24-round class): each item is loaded, reduced and
+// stored by twice the waves, but fewer items are resident at once.
+// Normalisation times, 4-wave / 8-wave: one clip 6.8 / 5.3 us, 40 ragged clips
+// 12.2 / 10.2, 10 min long form (47 chunks) 18.0 / 15.2, 64 x 15 s 20.3 /
+// 18.5, 1 h (280 chunks) 77 / 72, 8 h to bf16 436 / 428; but 128 clips of
+// 1-15 s 18.9 / 20.5, 256 of 1-20 s 50.2 / 52, 128 of 7.5-15 s 25.0 / 26.1:
+// once the items no longer fit at 3 per CU, the 8-wave form needs them of
+// nearly one length (measured down to 7/8 of the longest on average: 128 of
+// 11-15 s 30.6 / 30.1).
 constexpr int kNormWideWaves = 8;
-constexpr int kNormWideMaxItems = 16;
+constexpr int kNormWidePerCu = 3;
+inline bool norm_wide(int n_items, int max_T, int64_t sum_T, int cus) {
+  return (int64_t)n_items * kSlabs <= (int64_t)kNormWidePerCu * cus || 8 * sum_T >= (int64_t)7 * max_T * n_items;
+}
 
 template <int N, typename O>
 __global__ __launch_bounds__(64 * kNormWideWaves) void sfe_norm_wide_kernel(const float* __restrict__ raw,
@@ -1086,8 +1109,9 @@ hipError_t launch_logmel(const void* samples, int pcm, float pcm_scale, const It
 }
 
 template <typename O>
-hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int max_T, int pad_to, O* out, int n_segs,
-                         const int32_t* seg_item, double2* parts, hipStream_t stream) {
+hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, int cus,
+                         int pad_to, O* out, int n_segs, const int32_t* seg_item, double2* parts,
+                         hipStream_t stream) {
   using S = NormShape<kNormMainWaves>;
   using SW = NormShape<kNormWideWaves>;
   const unsigned blocks = (unsigned)((int64_t)n_items * kSlabs);
@@ -1103,9 +1127,11 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
                                                                                  out);
     return hipGetLastError();
   }
-  if (n_items <= kNormWideMaxItems) {
+  if (norm_wide(n_items, max_T, sum_T, cus)) {
     const dim3 grid(blocks), block(SW::kThreads);
     if (max_T <= SW::kSpan * 8) sfe_norm_wide_kernel<8, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
+    else if (max_T <= SW::kSpan * 12)
+      sfe_norm_wide_kernel<12, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
     else sfe_norm_wide_kernel<16, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
     return hipGetLastError();
   }
@@ -1119,13 +1145,16 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
   return hipGetLastError();
 }
 
-hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int pad_to, void* out,
-                       bool out_bf16, int n_segs, const int32_t* seg_item, void* parts, hipStream_t stream) {
+hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, int cus, int pad_to,
+                       void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
+                       hipStream_t stream) {
   if (n_items <= 0) return hipSuccess;
   double2* p = static_cast<double2*>(parts);
   if (out_bf16)
-    return launch_norm_t(raw, items, n_items, max_T, pad_to, static_cast<uint16_t*>(out), n_segs, seg_item, p, stream);
-  return launch_norm_t(raw, items, n_items, max_T, pad_to, static_cast<float*>(out), n_segs, seg_item, p, stream);
+    return launch_norm_t(raw, items, n_items, max_T, sum_T, cus, pad_to, static_cast<uint16_t*>(out), n_segs, seg_item,
+                         p, stream);
+  return launch_norm_t(raw, items, n_items, max_T, sum_T, cus, pad_to, static_cast<float*>(out), n_segs, seg_item, p,
+                       stream);
 }
 
 }  // namespace sfe

@@ -270,7 +270,8 @@ void sfe_logmel_kernel(const S* __restrict__ samples, const Item* __restrict__ i
   // Special columns: lane 4 j + n reads inputs 8 (j / 8) .. of frame n's row
   // 0, which holds (Y[0], Y[16]): Y[0] for j % 8 < 4.
   const float* xs = sb + kSlot * (lane & 3) + 16 * (lane >> 5) + ((lane >> 4) & 1);
-  // Power spectra [bin][frame]: bins l + 32 k2 and 32 m - l of frame g; this
+  // Power spectra [bin][frame] (bin 0 holds no power and is not read): bins l
+  // + 32 k2 and 32 m - l of frame g; this
   // lane's special bin of frame lane % 4 (after the halves are exchanged, h =
   // lane / 32).
   float* p_lo = sb + 4 * l + g;

@@ -63,7 +63,7 @@ void mel_filterbank(int n_fft, int n_mels, int sample_rate, float* out) {
 }
 
 namespace {
-// Chooses k0[j] in (hi[j] - S, lo[j]] with distinct k0[j] mod 16, as far as a
+// Chooses k0[j] >= 1 in (hi[j] - S, lo[j]] with distinct k0[j] mod 16, as far as a
 // matching (augmenting paths) finds one; the others keep lo[j].
 void spread_banks(const int (&lo)[16], const int (&hi)[16], int S, int (&k0)[16]) {
   int owner[16];  // bank group -> lane
@@ -76,7 +76,7 @@ void spread_banks(const int (&lo)[16], const int (&hi)[16], int S, int (&k0)[16]
     int (&owner)[16];
     bool seen[16];
     bool place(int j) {
-      for (int k = lo[j]; k >= 0 && k > hi[j] - S; --k) {
+      for (int k = lo[j]; k >= 1 && k > hi[j] - S; --k) {
         const int u = k % 16;
         if (seen[u]) continue;
         seen[u] = true;
@@ -176,11 +176,13 @@ bool build_dev_tables(int sample_rate, DevTables* t) {
         lo[j] = 0, hi[j] = kBins - 1;
         while (lo[j] < kBins && f[lo[j]] == 0.0f) ++lo[j];
         while (hi[j] > lo[j] && f[hi[j]] == 0.0f) --hi[j];
-        if (lo[j] == kBins) lo[j] = hi[j] = 0;  // an all-zero filter
+        if (lo[j] == kBins) lo[j] = hi[j] = 1;  // an all-zero filter
         lo[j] = std::min(lo[j], kBins - S);
         if (hi[j] >= lo[j] + S) return false;
         k0[j] = lo[j];
       }
+      // Bin 0 has no weight at any rate (0 Hz is the first filter's edge) and
+      // is never read: the kernel leaves it undefined.
       // 16 lanes' 16-byte reads of power bins fall on 16 groups of banks:
       // slot 1's filters are wider apart than the first bins of slot 0's,
       // which mostly share bins, so where the slot is wider than the filter

@@ -123,8 +123,10 @@ def featurize_long_form(extractor: ParakeetFeatureExtractor, recording, config: 
         raise EmptyAudio()
     if n <= cfg.transcription.max_audio_samples:
         table = np.array([[0, n, 0, 0]], np.int64)
-    else:
+    elif type(cfg.overlap) is OverlapChunkConfig:
         table = cfg.overlap._table(n)
+    else:  # a caller's own planner
+        table = TaskTable(build_fast_execution_plan(n, cfg)).array
     # (the call is enqueued first: the GPU works while the task list is made)
     out, fo = extractor.extract_chunks(recording, TaskTable(table, extractor.config.hop_length), dtype=dtype,
                                        stream=stream)

@@ -130,7 +130,7 @@ int main(int argc, char** argv) {
   check("low-energy bins of a loud tone, same scale", equiet, 1.0);
 
   // The mel schedule holds every nonzero weight of every filter exactly, and
-  // reads bins 0 .. 256 only.
+  // reads bins 1 .. 256 only.
   std::vector<float> fb((size_t)sfe::kMel * sfe::kBins);
   sfe::mel_filterbank(sfe::kNfft, sfe::kMel, rate, fb.data());
   double wrong = 0;
@@ -140,7 +140,7 @@ int main(int argc, char** argv) {
     for (int L = 0; L < 64; ++L) {
       std::vector<float> row(sfe::kBins, 0.0f);
       const int k0 = tb.mel_k0[i][L];
-      if (k0 < 0 || k0 + S > sfe::kBins) ++wrong;
+      if (k0 < 1 || k0 + S > sfe::kBins) ++wrong;
       else
         for (int s = 0; s < S; ++s)
           row[k0 + s] = reinterpret_cast<const float*>(&tb.mel_w[(first + s) / 4][L])[(first + s) % 4];

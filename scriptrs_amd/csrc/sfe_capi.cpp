@@ -169,11 +169,13 @@ struct PinBuf {
 // after every upload, waited for by the next call, cost each call a marker
 // between its upload and its first kernel (5.6 us on the device) and held the
 // host to one call ahead.  The calls of a context are ordered after each
-// other, also across streams, so the event covers the whole half.
+// other, also across streams, so the event covers the whole half.  A piece
+// larger than a half takes the whole buffer, waiting for it on both sides.
 struct PinRing {
   char* ptr = nullptr;
   size_t half = 0, at = 0;  // at: bytes used of the current half
   int cur = 0;
+  bool whole = false;         // the last piece spans both halves
   hipEvent_t ev[2] = {nullptr, nullptr};
   bool pending[2] = {false, false};
   hipError_t wait(int h) {
@@ -181,8 +183,8 @@ struct PinRing {
     pending[h] = false;
     return hipEventSynchronize(ev[h]);
   }
-  // Room for pieces of up to `bytes`.  Growing waits for the device: uploads
-  // from the old buffer may be queued on any stream.
+  // A buffer of at least `bytes`.  Growing waits for the device: uploads from
+  // the old one may be queued on any stream.
   hipError_t reserve(size_t bytes) {
     hipError_t e;
     for (int h = 0; h < 2; ++h)
@@ -190,7 +192,7 @@ struct PinRing {
         ev[h] = nullptr;
         return e;
       }
-    const size_t want = (std::max(bytes, (size_t)4096) + 255) / 256 * 256;
+    const size_t want = (std::max(bytes, (size_t)4096) + 511) / 512 * 256;  // a half
     if (want <= half) return hipSuccess;
     if (ptr) {
       if ((e = hipDeviceSynchronize()) != hipSuccess) return e;
@@ -206,6 +208,7 @@ struct PinRing {
     half = want;
     at = 0;
     cur = 0;
+    whole = false;
     pending[0] = pending[1] = false;
     return hipSuccess;
   }
@@ -218,9 +221,17 @@ struct PinRing {
     if (at + n > half) {
       if ((e = hipEventRecord(ev[cur], stream)) != hipSuccess) return e;
       pending[cur] = true;
+      if ((whole || n > half) && (e = wait(cur)) != hipSuccess) return e;
       cur ^= 1;
-      at = 0;
       if ((e = wait(cur)) != hipSuccess) return e;
+      at = 0;
+      whole = n > half;
+      if (whole) {
+        cur = 1;
+        at = half;  // full
+        *out = ptr;
+        return hipSuccess;
+      }
     }
     *out = ptr + (size_t)cur * half + at;
     at += n;
@@ -485,6 +496,7 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
   if (!same) {
     ctx->meta_items.clear();
     SFE_HIP(ctx->meta.reserve(mbytes + 16));
+    SFE_HIP(ctx->h_meta.reserve(2 * mbytes));
     char* stage = nullptr;
     SFE_HIP(ctx->h_meta.take(mbytes, stream, &stage));
     memcpy(stage, table.data(), tbytes);
@@ -925,7 +937,7 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
       SFE_HIP(sfe::noalloc_scratch(ctx->device, &na));
       ctx->noalloc = static_cast<unsigned char*>(na);
     }
-    if (ctx->h_meta.half <
+    if (2 * ctx->h_meta.half <
             entries * sizeof(Item) + (sfe::kMaxLogmelWaves + sfe::kNoAllocMaxSegs) * sizeof(int32_t) ||
         ctx->na_in.capacity() < (size_t)n)
       return fail(SFE_HIP_ERROR, "context has no reserved planner buffers");

@@ -42,6 +42,7 @@
 #include "sfe_fft.hpp"
 #include "sfe_internal.hpp"
 #include "sfe_pcm.hpp"
+#include "sfe_seqsum.hpp"
 
 namespace sfe {
 
@@ -510,20 +511,23 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   return (uint16_t)(u >> 16);
 }
 
-// Statistics of a row whose values are all bitwise equal to x0.  This is
-// where the reference's sequential f32 sums decide the result: their
-// rounding leaves x - mean != 0 (about +-0.93 for digital silence), so the
-// sums are replayed on one lane in the reference's order
-// (src/frontend.rs:230-236).
+// Statistics of a row whose values are all bitwise equal to x0: digital
+// silence, and at sample rates past 24 kHz every row of a filter so narrow that
+// it holds no bin.  This is where the reference's sequential f32 sums decide
+// the result: their rounding leaves x - mean != 0 (about +-0.93 for digital
+// silence), so the sums are those of its loops (src/frontend.rs:230-236).
+//
+// What bounds it: a serial chain on one lane, while the rest of the workgroup
+// waits, in every workgroup of a long item (norm_finish).  Walking the row is
+// 2 T dependent additions, a sequential_sum about 4 per doubling of T.  Calls
+// with the rows walked / as sequential sums: 24 silent clips of 90 s 1200 /
+// 164 us (406 when one workgroup normalised a whole long item), 8 of 15 s 63 /
+// 28, 64 clips of 480,000 samples at 48 kHz 406 / 140.
 __device__ __forceinline__ void constant_row_stats(float x0, int T, float* mean_out, float* sd_out) {
 #pragma clang fp contract(off)  // every f32 operation rounded, as the reference's
-  float sum = 0.0f;
-  for (int t = 0; t < T; ++t) sum = sum + x0;
-  const float mean = __fdiv_rn(sum, (float)T);
+  const float mean = __fdiv_rn(sequential_sum(x0, T), (float)T);
   const float d = x0 - mean;
-  float acc = 0.0f;
-  for (int t = 0; t < T; ++t) acc = acc + d * d;
-  const float var = __fdiv_rn(acc, (float)T - 1.0f);
+  const float var = __fdiv_rn(sequential_sum(d * d, T), (float)T - 1.0f);
   *mean_out = mean;
   *sd_out = __fsqrt_rn(var) + 1e-5f;
 }

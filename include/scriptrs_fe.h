@@ -265,7 +265,7 @@ int sfe_extract_chunks_streamed_pcm(sfe_ctx* ctx, const void* host_recording, in
 /* Shared frames: on by default.  Overlapping chunk tasks of one call
  * (sfe_extract_chunks, _pcm, _padded, sfe_extract_batch; in the streamed
  * entry points, the tasks of one batch of windows) whose starts agree
- * modulo 4 hops have identical log-mel for a frame whose 512 padded
+ * modulo the hop have identical log-mel for a frame whose 512 padded
  * samples lie, in every task that holds it, after the task's first sample
  * and before its end; such frames are computed once and each task keeps
  * its first and last 4-frame groups.  The output is bitwise the same either

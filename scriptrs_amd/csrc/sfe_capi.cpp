@@ -414,9 +414,11 @@ int launch_pair(sfe_ctx* ctx, const Source& src, const Item* lm, const Item* d_l
   const int u1 = n_lm > 0 ? lm[n_lm - 1].unit_off + lm[n_lm - 1].n_units : 0;
   int max_T = 0;
   int64_t sum_T = 0;
+  bool shifted = false;
   for (int i = 0; i < n_norm; ++i) {
     max_T = std::max(max_T, (int)norm[i].T);
     sum_T += norm[i].T;
+    shifted |= norm[i].gshift % sfe::kQuad != 0;
   }
   hipEvent_t e[4] = {nullptr, nullptr, nullptr, nullptr};
   if (ctx->timing && allow_timing)
@@ -429,8 +431,8 @@ int launch_pair(sfe_ctx* ctx, const Source& src, const Item* lm, const Item* d_l
   if (e[1]) SFE_HIP(hipEventRecord(e[1], stream));
   if (e[2]) SFE_HIP(hipEventRecord(e[2], stream));
   if (stages & kNorm)
-    SFE_HIP(sfe::launch_norm(raw, d_norm, n_norm, max_T, sum_T, ctx->cus, pad_to, out, out_dtype == SFE_BF16, segs.n,
-                             segs.d_item, segs.parts, stream));
+    SFE_HIP(sfe::launch_norm(raw, d_norm, n_norm, max_T, sum_T, shifted, ctx->cus, pad_to, out,
+                             out_dtype == SFE_BF16, segs.n, segs.d_item, segs.parts, stream));
   if (e[3]) SFE_HIP(hipEventRecord(e[3], stream));
   return SFE_OK;
 }

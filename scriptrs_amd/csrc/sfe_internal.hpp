@@ -58,8 +58,8 @@ __host__ __device__ constexpr int64_t raw_frame(int64_t f) { return raw_quad(f >
 // log-mel is read from raw[grid_off + raw_frame(f + gshift)] for f in
 // [f_lo, f_hi], raw[tail_off + raw_frame(f)] past f_hi and raw[out_off +
 // raw_frame(f)] below f_lo.  An item with its own region has f_lo = 0,
-// f_hi = T - 1, grid_off = out_off and gshift = 0.  Else f_lo, f_hi + 1 and
-// gshift are multiples of 4: the regions meet at whole quads of the item.
+// f_hi = T - 1, grid_off = out_off and gshift = 0.  Else f_lo and f_hi + 1 are
+// multiples of 4: the regions meet at whole quads of the item.
 struct Item {
   int64_t start;
   int64_t len;
@@ -96,9 +96,9 @@ inline Item own_item(int64_t start, int64_t len, int64_t out_off, int64_t dst_of
 }
 
 // Shared frames (sfe_share.cpp).  Frames of overlapping items whose samples
-// lie at least one sample inside each item and whose starts agree modulo 4
-// hops (one quad) are computed once: items' own regions keep only their first
-// quad and their last quads, and a shared log-mel entry per run of such items covers
+// lie at least one sample inside each item and whose starts agree modulo the
+// hop are computed once: items' own regions keep only their first quad and
+// their last quads, and a shared log-mel entry per run of such items covers
 // the union of their interior frames.  Given items with their own regions
 // (own_item; out_off ignored), plan_table fills one table, table[0, *n_lm)
 // with the log-mel entries and table[*n_lm, *n_lm + n) with the
@@ -110,7 +110,7 @@ constexpr int kPlanEntriesPerItem = 3;  // log-mel entries per item at most
 struct PlanWorkspace {
   struct Span {
     int idx;              // item index
-    int64_t res, lo, hi;  // start mod 4 hops; interior frames in recording frame indices
+    int64_t res, lo, hi;  // start mod hop; interior frames in recording frame indices
   };
   struct Run {
     int64_t res, lo, hi;   // union of interior frames (recording frame indices)
@@ -281,12 +281,12 @@ hipError_t launch_logmel(const void* samples, int pcm, float pcm_scale, const It
 // and writes feature-major [128][T] per item to out (f32, must not alias
 // raw) or bf16 (uint16_t*) when out_bf16 is set.  max_T: the longest item's
 // frame count (sizes the kernel's register budget); sum_T: all items' frames;
-// cus: the device's compute units.  pad_to > 0: rows of
-// pad_to frames, zero past T (the encoder input layout).  n_segs, seg_item,
-// parts: the long items' segments (norm_segments over items), the device copy
+// shifted: whether any item has gshift % kQuad != 0; cus: the device's
+// compute units.  pad_to > 0: rows of pad_to frames, zero past T (the encoder
+// input layout).  n_segs, seg_item, parts: the long items' segments (norm_segments over items), the device copy
 // of their entry indexes and n_segs * kSegPartBytes of scratch.
-hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, int cus, int pad_to,
-                       void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
+hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, bool shifted,
+                       int cus, int pad_to, void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
                        hipStream_t stream);
 
 // Static scratch of the allocation-free entry point (sfe_noalloc.hip): an

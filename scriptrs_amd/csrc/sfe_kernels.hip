@@ -38,10 +38,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "sfe_fft.hpp"
 #include "sfe_internal.hpp"
 #include "sfe_pcm.hpp"
+#include "sfe_rounds.hpp"
 #include "sfe_seqsum.hpp"
 
 namespace sfe {
@@ -572,12 +574,24 @@ struct NormShape {
   static_assert(4 * kLanesPerRow == kSpan, "a store instruction covers one round of a row");
 };
 
+// A normalisation workgroup's LDS.  Two transpose buffers in the 4-wave form
+// (chunk ch stages into tb[ch % 2]: the next chunk's staging does not wait for
+// this chunk's stores, one barrier per chunk); one in the 8-wave form, whose
+// buffer is twice as large.
+constexpr int kSumParts = 8;
+template <int W>
+struct NormLds {
+  static constexpr int kTBufs = W == 4 ? 2 : 1;
+  double red[kSumParts * kSlabF];
+  float st[3 * kSlabF];
+  __attribute__((aligned(16))) float tb[kTBufs][kSlabF * NormShape<W>::kTStride];
+};
+
 // Workgroup sum over the lanes that hold the same feature (lane % 16 equal)
 // and the waves; every lane gets its own feature's total.  v[k] holds the
 // lane's sum over rounds j = k mod 8 / W: tile 4 j + w of a 4-wave workgroup is
 // tile 8 (j / 2) + w + 4 (j % 2) of an 8-wave one, so both add the same 8 sums
 // in the same order and the results do not depend on the form.
-constexpr int kSumParts = 8;
 template <int W>
 __device__ __forceinline__ double slab_sum(double (&v)[kSumParts / W], double* red, int lane, int w) {
 #pragma unroll
@@ -672,54 +686,40 @@ __device__ __forceinline__ void zero_tail(O* __restrict__ ob, int T, int rs, int
   for (int e = w * 64 + lane; e < kSlabF * tail; e += W * 64) put1(ob + (size_t)(e / tail) * rs + T + e % tail, 0.0f);
 }
 
-// Where a normalisation workgroup's lane finds its quads: round j holds quad
-// q + 4 W j of the item (q counts from quad q0, a multiple of 4, where the
-// workgroup starts), at byte off(j) from the uniform base (the tile of the
-// item's shared frames where the workgroup starts, this slab).  An item's own first quad and last
-// tiles come after its shared region (at most kMaxShareFrames frames, then at
-// most 3 tiles for each of at most kMaxShareMembers members), so 32-bit byte
-// offsets reach them; an item with its own region has all three at out_off.
-// The region is chosen by adding differences under conditions (a choice among
-// several values compiles to a table in private memory).
-template <int W>
-struct Rounds {
-  const char* base;
-  uint32_t og, dlo, dhi;
-  int q;         // the lane's quad in round 0
-  int qlo, qhi;  // quads [qlo, qhi] are in the shared region
-  int left;      // T - 4 q: element e of round j is inside the item where 16 W j + e < left
-  static constexpr uint32_t kRound = 4u * kRawTile * W;  // bytes
-
-  __device__ __forceinline__ Rounds(const float* raw, const Item& it, int slab, int lane, int w, int q0) {
-    const int gs = it.gshift / kQuad;
-    const int tile0 = (q0 + gs) & ~3;  // quad of the shared region at the base: offsets stay small in any item
-    base = reinterpret_cast<const char*>(raw + it.grid_off + raw_quad(tile0) + kRawSlab * slab);
-    q = q0 + 4 * w + (lane >> 4);
-    og = 4u * (uint32_t)(raw_quad(q + gs - tile0) + 4 * (lane & 15));
-    const int64_t own = raw_quad(q) - raw_quad(q + gs) - it.grid_off;
-    dlo = 4u * (uint32_t)(it.out_off + own);
-    dhi = 4u * (uint32_t)(it.tail_off + own);
-    qlo = it.f_lo / kQuad;
-    qhi = it.f_hi / kQuad;
-    left = it.T - kQuad * q;
+// The lane's N quads (Rounds): raw buffer loads from the uniform base, all
+// issued before any is used (a load under a per-lane branch would wait for
+// itself).  One 16-byte load a quad where the item's quads are quads of its
+// regions (SHIFT = 0); the 4 - SHIFT frames from one quad of the shared region
+// and the SHIFT from the next in two loads where it starts inside one.
+template <int SHIFT, int W, int N>
+__device__ __forceinline__ void load_rounds(const Rounds<W>& rd, float4 (&v)[N]) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x3 __attribute__((ext_vector_type(3)));
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(rd.base), 0, kNormBufRange, kBufWord3);
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if constexpr (SHIFT == 0) {
+      v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
+    } else {
+      const int o0 = rd.template elem_off<SHIFT>(j, 0), o1 = rd.template elem_off<SHIFT>(j, kQuad - SHIFT);
+      if constexpr (SHIFT == 1) {
+        const f32x3 a = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(rsrc, o0, 0, 0));
+        const float b = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o1, 0, 0));
+        v[j] = make_float4(a.x, a.y, a.z, b);
+      } else if constexpr (SHIFT == 2) {
+        const f32x2 a = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, o0, 0, 0));
+        const f32x2 b = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, o1, 0, 0));
+        v[j] = make_float4(a.x, a.y, b.x, b.y);
+      } else {
+        const float a = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, o0, 0, 0));
+        const f32x3 b = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(rsrc, o1, 0, 0));
+        v[j] = make_float4(a, b.x, b.y, b.z);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one round's addresses at a time: they take registers beside v
+    }
   }
-  __device__ __forceinline__ uint32_t off(int j) const {
-    uint32_t o = og + kRound * (uint32_t)j + (q + 4 * W * j > qhi ? dhi : 0u);
-    if (j == 0) o += q < qlo ? dlo : 0u;  // (the own first quad is quad 0)
-    return o;
-  }
-  // Past the item: an offset past the buffer's range, for which the hardware
-  // returns zeros without a memory access.
-  __device__ __forceinline__ int buf_off(int j) const {
-    return 16 * W * j < left ? (int)off(j) : kNormBufRange;
-  }
-  // Whether every lane of the workgroup holds 4 frames of the item in round j,
-  // T frames counted from the workgroup's first.
-  static __device__ __forceinline__ bool full(int j, int T) { return 16 * W * (j + 1) <= T; }
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer() const {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, kNormBufRange, kBufWord3);
-  }
-};
+}
 
 // Adds the f32 sum over a quad of (x - p) to s; elements past the item (index >= n)
 // left out.  (all is uniform and rarely false: an empty asm keeps the masked
@@ -755,23 +755,17 @@ __device__ __forceinline__ void add_sq(double& s, const float4& v, float p, bool
 // in registers and read once.  Every N sums the same quads, so the class does
 // not change the result.  `work` is the (item, slab) index; items longer than
 // kNormRegFrames are left to norm_segment and norm_finish.
-template <int W, int N, typename O>
-__device__ __forceinline__ void norm_body(const float* __restrict__ raw, const Item* __restrict__ items,
-                                          int n_items, int work, int pad_to, O* __restrict__ out) {
+template <int SHIFT, int W, int N, typename O>
+__device__ __forceinline__ void norm_body(const float* __restrict__ raw, const Item* __restrict__ items, int work,
+                                          int pad_to, O* __restrict__ out, NormLds<W>& lds) {
   static_assert(N % 4 == 0, "whole chunks");
   using S = NormShape<W>;
   constexpr int kSpan = S::kSpan;
   constexpr int kChunk = S::kChunk;
-  __shared__ double red[kSumParts * kSlabF];
-  __shared__ float st[3 * kSlabF];
-  // Two transpose buffers in the 4-wave form (chunk ch stages into tb[ch %
-  // 2]: the next chunk's staging does not wait for this chunk's stores, one
-  // barrier per chunk); one in the 8-wave form, whose buffer is twice as
-  // large.
-  constexpr int kTBufs = W == 4 ? 2 : 1;
-  __shared__ __align__(16) float tb[kTBufs][kSlabF * S::kTStride];
+  constexpr int kTBufs = NormLds<W>::kTBufs;
+  double* red = lds.red;
+  float* st = lds.st;
   const int item = work / kSlabs;
-  if (item >= n_items) return;
 #ifdef SFE_TIMESTAMPS
   const int64_t sn = kStampNorm + 4 * (int64_t)work;
   if (threadIdx.x == 0) SFE_STAMP(sn, stamp_now());
@@ -798,12 +792,7 @@ __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const I
   constexpr int K = kSumParts / W;
   double sp[K] = {}, qp[K] = {};
   float4 v[N];
-  // Raw buffer loads from the uniform base, all issued before any is used
-  // (a load under a per-lane branch would wait for itself).
-  const __amdgpu_buffer_rsrc_t rsrc = rd.buffer();
-#pragma unroll
-  for (int j = 0; j < N; ++j)
-    v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
+  load_rounds<SHIFT>(rd, v);
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     v[j] = ln2_scale(v[j]);
@@ -824,7 +813,7 @@ __device__ __forceinline__ void norm_body(const float* __restrict__ raw, const I
 #pragma unroll
   for (int ch = 0; ch < N / 4; ++ch) {
     if (ch < chunks) {
-      float* t = tb[ch % kTBufs];
+      float* t = lds.tb[ch % kTBufs];
 #pragma unroll
       for (int jr = 0; jr < 4; ++jr) stage(t, jr, v[4 * ch + jr]);
       __syncthreads();
@@ -855,9 +844,27 @@ constexpr int kNormMainWaves = 4;
 
 template <int N, typename O>
 __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_kernel(const float* __restrict__ raw,
-                                                                       const Item* __restrict__ items, int n_items,
-                                                                       int pad_to, O* __restrict__ out) {
-  norm_body<kNormMainWaves, N>(raw, items, n_items, blockIdx.x, pad_to, out);
+                                                                       const Item* __restrict__ items, int pad_to,
+                                                                       O* __restrict__ out) {
+  __shared__ NormLds<kNormMainWaves> lds;
+  norm_body<0, kNormMainWaves, N>(raw, items, blockIdx.x, pad_to, out, lds);
+}
+
+// Runs body<shift> for the item's own shift: one instance a value, each with
+// its loads and nothing to choose per load.  (Chosen inside one instance, the
+// loads of all four forms meet in the same registers, which took 107 a lane
+// instead of 74 in the 12-round class.)  716 windows of 15 s every 5.01 s: 152
+// us, against 144 on a grid of 4 hops (5.00 s); four 4-byte loads a quad, for
+// any shift, took 222.  The call, whose log-mel is then one shared region
+// instead of one per residue, 501 -> 265 us; 1 h in windows of 15 s every 13.01
+// s 195 -> 180.
+template <bool SHIFT, class F>
+__device__ __forceinline__ void with_shift(const Item& it, F&& body) {
+  const int s = SHIFT ? it.gshift % kQuad : 0;
+  if (s == 0) body(std::integral_constant<int, 0>());
+  else if (s == 1) body(std::integral_constant<int, 1>());
+  else if (s == 2) body(std::integral_constant<int, 2>());
+  else body(std::integral_constant<int, 3>());
 }
 
 // Long items, in segments of seg_frames(T) frames, chunks of 512 in registers.
@@ -878,12 +885,13 @@ __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_kernel(const flo
 // are read once, and 256 clips of 1-20 s take 49 us.
 constexpr int kSegRounds = kSegFrames / (kTile * kNormMainWaves);
 
+template <int SHIFT>
 __device__ __forceinline__ void norm_segment(const float* __restrict__ raw, const Item* __restrict__ items,
                                              const int32_t* __restrict__ seg_item, int work,
-                                             double2* __restrict__ parts) {
+                                             double2* __restrict__ parts, NormLds<kNormMainWaves>& lds) {
   constexpr int W = kNormMainWaves;
   constexpr int kSpan = NormShape<W>::kSpan;
-  __shared__ double red[kSumParts * kSlabF];
+  double* red = lds.red;
   const int seg = work / kSlabs, slab = work % kSlabs;
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
@@ -895,11 +903,8 @@ __device__ __forceinline__ void norm_segment(const float* __restrict__ raw, cons
   for (int t = t0; t < t1; t += kSegFrames) {
     const int n = t1 - t < kSegFrames ? t1 - t : kSegFrames;
     const Rounds<W> rd(raw, it, slab, lane, w, t / kQuad);
-    const __amdgpu_buffer_rsrc_t rsrc = rd.buffer();
     float4 v[kSegRounds];
-#pragma unroll
-    for (int j = 0; j < kSegRounds; ++j)
-      v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
+    load_rounds<SHIFT>(rd, v);
     constexpr int K = kSumParts / W;
     double sp[K] = {}, qp[K] = {};
 #pragma unroll
@@ -919,15 +924,15 @@ __device__ __forceinline__ void norm_segment(const float* __restrict__ raw, cons
   if (w == 0 && lane < kSlabF) parts[(size_t)work * kSlabF + lane] = make_double2(S, V);
 }
 
-template <typename O>
+template <int SHIFT, typename O>
 __device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const Item* __restrict__ items,
                                             const int32_t* __restrict__ seg_item, int work,
-                                            const double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
+                                            const double2* __restrict__ parts, int pad_to, O* __restrict__ out,
+                                            NormLds<kNormMainWaves>& lds) {
   constexpr int W = kNormMainWaves;
   using NS = NormShape<W>;
-  __shared__ double red[kSumParts * kSlabF];
-  __shared__ float st[3 * kSlabF];
-  __shared__ __align__(16) float tb[2][kSlabF * NS::kTStride];
+  double* red = lds.red;
+  float* st = lds.st;
   const int seg = work / kSlabs, slab = work % kSlabs;
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
@@ -940,13 +945,7 @@ __device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const
   if (pad_to > 0 && t1 == T) zero_tail<W>(ob, T, rs, lane, w);
   const float x0 = ln2_scale(raw[it.out_off + kRawSlab * slab + 4 * (lane & 15)]);
   float4 v[kSegRounds];
-  auto load = [&](int t) {
-    const Rounds<W> rd(raw, it, slab, lane, w, t / kQuad);
-    const __amdgpu_buffer_rsrc_t rsrc = rd.buffer();
-#pragma unroll
-    for (int j = 0; j < kSegRounds; ++j)
-      v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, rd.buf_off(j), 0, 0));
-  };
+  auto load = [&](int t) { load_rounds<SHIFT>(Rounds<W>(raw, it, slab, lane, w, t / kQuad), v); };
   load(t0);
   // Segment k of the item: wave k % 4, lanes 16 (k / 4 % 4) ..
   double Sp[kSumParts / W] = {}, Vp[kSumParts / W] = {};
@@ -965,30 +964,38 @@ __device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const
     for (int ch = 0; ch < kSegRounds / 4; ++ch) {
 #pragma unroll
       for (int jr = 0; jr < 4; ++jr)
-        *reinterpret_cast<float4*>(tb[ch % 2] + (lane & 15) * NS::kTStride + NS::kSpan * jr + 16 * w +
+        *reinterpret_cast<float4*>(lds.tb[ch % 2] + (lane & 15) * NS::kTStride + NS::kSpan * jr + 16 * w +
                                    kQuad * (lane >> 4)) = ln2_scale(v[4 * ch + jr]);
       __syncthreads();
-      store_chunk<W>(tb[ch % 2], st, t + NS::kChunk * ch, t1, rs, lane, w, ob);
+      store_chunk<W>(lds.tb[ch % 2], st, t + NS::kChunk * ch, t1, rs, lane, w, ob);
     }
   }
 }
 
 // Workgroups [0, 8 n_segs): the long items' segments; the rest normalise the
 // other items.
-template <int N, typename O>
+template <bool SHIFT, int N, typename O>
 __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_long_kernel(
-    const float* __restrict__ raw, const Item* __restrict__ items, int n_items, int n_segs,
-    const int32_t* __restrict__ seg_item, double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
-  const int b = blockIdx.x;
-  if (b < kSlabs * n_segs) norm_segment(raw, items, seg_item, b, parts);
-  else norm_body<kNormMainWaves, N>(raw, items, n_items, b - kSlabs * n_segs, pad_to, out);
+    const float* __restrict__ raw, const Item* __restrict__ items, int n_segs, const int32_t* __restrict__ seg_item,
+    double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
+  __shared__ NormLds<kNormMainWaves> lds;
+  const int b = blockIdx.x, rest = b - kSlabs * n_segs;
+  if (rest < 0)
+    with_shift<SHIFT>(items[seg_item[b / kSlabs]],
+                      [&](auto s) { norm_segment<s()>(raw, items, seg_item, b, parts, lds); });
+  else
+    with_shift<SHIFT>(items[rest / kSlabs],
+                      [&](auto s) { norm_body<s(), kNormMainWaves, N>(raw, items, rest, pad_to, out, lds); });
 }
 
-template <typename O>
+template <bool SHIFT, typename O>
 __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_finish_kernel(
     const float* __restrict__ raw, const Item* __restrict__ items, const int32_t* __restrict__ seg_item,
     const double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
-  norm_finish(raw, items, seg_item, blockIdx.x, parts, pad_to, out);
+  __shared__ NormLds<kNormMainWaves> lds;
+  const int b = blockIdx.x;
+  with_shift<SHIFT>(items[seg_item[b / kSlabs]],
+                    [&](auto s) { norm_finish<s()>(raw, items, seg_item, b, parts, pad_to, out, lds); });
 }
 
 // 8-wave workgroups (128 frames per round, 33 KB of LDS for the 512-frame
@@ -1008,12 +1015,14 @@ inline bool norm_wide(int n_items, int max_T, int64_t sum_T, int cus) {
   return (int64_t)n_items * kSlabs <= (int64_t)kNormWidePerCu * cus || 8 * sum_T >= (int64_t)7 * max_T * n_items;
 }
 
-template <int N, typename O>
+template <bool SHIFT, int N, typename O>
 __global__ __launch_bounds__(64 * kNormWideWaves) void sfe_norm_wide_kernel(const float* __restrict__ raw,
                                                                             const Item* __restrict__ items,
-                                                                            int n_items, int pad_to,
-                                                                            O* __restrict__ out) {
-  norm_body<kNormWideWaves, N>(raw, items, n_items, blockIdx.x, pad_to, out);
+                                                                            int pad_to, O* __restrict__ out) {
+  __shared__ NormLds<kNormWideWaves> lds;
+  const int b = blockIdx.x;
+  with_shift<SHIFT>(items[b / kSlabs],
+                    [&](auto s) { norm_body<s(), kNormWideWaves, N>(raw, items, b, pad_to, out, lds); });
 }
 
 }  // namespace
@@ -1113,7 +1122,7 @@ hipError_t launch_logmel(const void* samples, int pcm, float pcm_scale, const It
                                       raw_out, g.blocks, wave_item, stream);
 }
 
-template <typename O>
+template <bool SHIFT, typename O>
 hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, int cus,
                          int pad_to, O* out, int n_segs, const int32_t* seg_item, double2* parts,
                          hipStream_t stream) {
@@ -1124,42 +1133,48 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
     // Long items among them: their segments' sums beside the other items,
     // then the segments themselves.
     const unsigned seg_blocks = (unsigned)((int64_t)n_segs * kSlabs);
-    sfe_norm_long_kernel<kNormRegFrames / S::kSpan, O><<<dim3(seg_blocks + blocks), dim3(S::kThreads), 0, stream>>>(
-        raw, items, n_items, n_segs, seg_item, parts, pad_to, out);
+    sfe_norm_long_kernel<SHIFT, kNormRegFrames / S::kSpan, O>
+        <<<dim3(seg_blocks + blocks), dim3(S::kThreads), 0, stream>>>(raw, items, n_segs, seg_item, parts, pad_to,
+                                                                      out);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    sfe_norm_finish_kernel<O><<<dim3(seg_blocks), dim3(S::kThreads), 0, stream>>>(raw, items, seg_item, parts, pad_to,
-                                                                                 out);
+    sfe_norm_finish_kernel<SHIFT, O><<<dim3(seg_blocks), dim3(S::kThreads), 0, stream>>>(raw, items, seg_item, parts,
+                                                                                        pad_to, out);
     return hipGetLastError();
   }
-  if (norm_wide(n_items, max_T, sum_T, cus)) {
+  // (SHIFT has no 4-wave kernels: tasks that share frames are mostly of one
+  // length, where the 8-wave form is the faster one, and it loses 4% at most)
+  if (SHIFT || norm_wide(n_items, max_T, sum_T, cus)) {
     const dim3 grid(blocks), block(SW::kThreads);
-    if (max_T <= SW::kSpan * 8) sfe_norm_wide_kernel<8, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
+    if (max_T <= SW::kSpan * 8)
+      sfe_norm_wide_kernel<SHIFT, 8, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
     else if (max_T <= SW::kSpan * 12)
-      sfe_norm_wide_kernel<12, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
-    else sfe_norm_wide_kernel<16, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
+      sfe_norm_wide_kernel<SHIFT, 12, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
+    else
+      sfe_norm_wide_kernel<SHIFT, 16, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
     return hipGetLastError();
   }
   const dim3 grid(blocks), block(S::kThreads);
   // Registers per lane sized to the longest item (N float4s hold kSpan N
   // frames).
-  if (max_T <= S::kSpan * 8) sfe_norm_kernel<8, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
-  else if (max_T <= S::kSpan * 16) sfe_norm_kernel<16, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
-  else if (max_T <= S::kSpan * 24) sfe_norm_kernel<24, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
-  else sfe_norm_kernel<32, O><<<grid, block, 0, stream>>>(raw, items, n_items, pad_to, out);
+  if (max_T <= S::kSpan * 8) sfe_norm_kernel<8, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
+  else if (max_T <= S::kSpan * 16) sfe_norm_kernel<16, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
+  else if (max_T <= S::kSpan * 24) sfe_norm_kernel<24, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
+  else sfe_norm_kernel<32, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
   return hipGetLastError();
 }
 
-hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, int cus, int pad_to,
-                       void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
+hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, bool shifted,
+                       int cus, int pad_to, void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
                        hipStream_t stream) {
   if (n_items <= 0) return hipSuccess;
   double2* p = static_cast<double2*>(parts);
-  if (out_bf16)
-    return launch_norm_t(raw, items, n_items, max_T, sum_T, cus, pad_to, static_cast<uint16_t*>(out), n_segs, seg_item,
-                         p, stream);
-  return launch_norm_t(raw, items, n_items, max_T, sum_T, cus, pad_to, static_cast<float*>(out), n_segs, seg_item, p,
-                       stream);
+  auto go = [&](auto* o) {
+    return shifted ? launch_norm_t<true>(raw, items, n_items, max_T, sum_T, cus, pad_to, o, n_segs, seg_item, p, stream)
+                   : launch_norm_t<false>(raw, items, n_items, max_T, sum_T, cus, pad_to, o, n_segs, seg_item, p,
+                                          stream);
+  };
+  return out_bf16 ? go(static_cast<uint16_t*>(out)) : go(static_cast<float*>(out));
 }
 
 }  // namespace sfe

@@ -16,13 +16,13 @@
 // Per item of T frames, frames 2 to (len - kPad) / hop are its own samples
 // alone: frame f's 512 padded samples (item samples 160 f - 256 .. 160 f +
 // 255) then lie in [1, len).  The interior frames are the whole quads among
-// them, from frame 4 on.  Items whose starts agree modulo 4 hops (so that
-// their quads coincide) and whose interior frames overlap or touch form a
-// run; a run's shared log-mel entry
+// them, from frame 4 on.  Items whose starts agree modulo the hop and whose
+// interior frames overlap or touch form a run; a run's shared log-mel entry
 // spans the samples from its first item's start to its last item's end and
-// covers the union of their interior frames.  Each item keeps its own first
-// quad (frames 0-3) and its last quads (frames past the interior), in tiles
-// of its own.  A run is shared only if that computes fewer quads than its
+// covers the union of their interior frames.  (An item that starts inside a
+// quad of the shared region finds its own quads across two of them,
+// Rounds::elem_off.)  Each item keeps its own first quad (frames 0-3) and its
+// last quads (frames past the interior), in tiles of its own.  A run is shared only if that computes fewer quads than its
 // items would alone.
 #include <algorithm>
 #include <vector>
@@ -34,7 +34,6 @@ namespace sfe {
 namespace {
 
 constexpr int kShareLo = kQuad;   // first interior frame
-constexpr int64_t kShareGrid = (int64_t)kQuad * kHop;
 constexpr int kMinInterior = 32;  // fewer interior frames: the item keeps its own region
 
 int interior_hi(const Item& it) { return (int)(((it.len - kPad) / kHop + 1) / kQuad * kQuad - 1); }
@@ -65,7 +64,7 @@ int64_t plan_table(const Item* items, int n, bool share, PlanWorkspace* ws, Item
       const int hi = interior_hi(it);
       if (hi - kShareLo + 1 < kMinInterior) continue;
       const int64_t c = it.start / kHop;
-      sp.push_back({i, it.start % kShareGrid, c + kShareLo, c + hi});
+      sp.push_back({i, it.start % kHop, c + kShareLo, c + hi});
     }
     std::sort(sp.begin(), sp.end(), [](const PlanWorkspace::Span& a, const PlanWorkspace::Span& b) {
       return a.res != b.res ? a.res < b.res : (a.lo != b.lo ? a.lo < b.lo : a.idx < b.idx);

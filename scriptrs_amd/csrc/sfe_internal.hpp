@@ -219,6 +219,19 @@ int64_t units_for(int64_t T);  // quads of an item: ceil(T / 4)
 constexpr int kPcmF32 = 0;
 constexpr int kPcmI16 = 1;
 constexpr int kPcmI32 = 2;
+// A launch holds fewer than 2^32 threads: `blocks` workgroups of `threads` go
+// in launches of at most that, in multiples of 8 workgroups.  go(first, n)
+// launches workgroups [first, first + n).
+template <class F>
+hipError_t for_launches(int64_t blocks, int threads, F&& go) {
+  const int64_t most = UINT32_MAX / threads / 8 * 8;
+  for (int64_t first = 0; first < blocks; first += most) {
+    const hipError_t e = go(first, (unsigned)(blocks - first < most ? blocks - first : most));
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 // Copies bytes (rounded up to 16; both sides 16-byte aligned and with room for
 // that) from pinned host memory to the device with a kernel on `stream`.
 hipError_t launch_upload(const void* src, void* dst, size_t bytes, hipStream_t stream);

@@ -52,15 +52,15 @@ __device__ __forceinline__ float vad_sample(const S* x, int64_t len, int64_t i, 
 }
 
 // One workgroup writes kVadRowsPerBlock model inputs, thread t float4 t of
-// them, so a wave's loads and stores are contiguous except across a row
-// boundary.  STREAM: nontemporal loads.
+// them (from row0), so a wave's loads and stores are contiguous except across a
+// row boundary.  STREAM: nontemporal loads.
 template <typename S, bool STREAM>
 __global__ __launch_bounds__(kVadThreads) void sfe_vad_frames_kernel(const S* __restrict__ x, int64_t len,
-                                                                     int64_t n_windows, Decode dc,
+                                                                     int64_t row0, int64_t n_windows, Decode dc,
                                                                      float* __restrict__ out) {
   const int r = (int)threadIdx.x / kVadRowVec;
   const int p = 4 * ((int)threadIdx.x - r * kVadRowVec);
-  const int64_t w = (int64_t)blockIdx.x * kVadRowsPerBlock + r;
+  const int64_t w = row0 + (int64_t)blockIdx.x * kVadRowsPerBlock + r;
   if (w >= n_windows) return;
   const int64_t i = w * kVadWin - kVadCtx + p;
   float4 v;
@@ -79,13 +79,17 @@ __global__ __launch_bounds__(kVadThreads) void sfe_vad_frames_kernel(const S* __
 }
 
 template <typename S>
-void launch_vad(const void* samples, int64_t len, int64_t n, const Decode& dc, float* out, hipStream_t stream) {
-  const dim3 g((unsigned)((n + kVadRowsPerBlock - 1) / kVadRowsPerBlock)), b(kVadThreads);
+hipError_t launch_vad(const void* samples, int64_t len, int64_t n, const Decode& dc, float* out, hipStream_t stream) {
   const S* x = static_cast<const S*>(samples);
-  if (sizeof(S) == 4 && 4 * (len + kVadRow * n) > kVadStreamBytes)
-    sfe_vad_frames_kernel<S, true><<<g, b, 0, stream>>>(x, len, n, dc, out);
-  else
-    sfe_vad_frames_kernel<S, false><<<g, b, 0, stream>>>(x, len, n, dc, out);
+  const bool streamed = sizeof(S) == 4 && 4 * (len + kVadRow * n) > kVadStreamBytes;
+  return for_launches((n + kVadRowsPerBlock - 1) / kVadRowsPerBlock, kVadThreads, [&](int64_t first, unsigned blocks) {
+    const int64_t row0 = first * kVadRowsPerBlock;
+    if (streamed)
+      sfe_vad_frames_kernel<S, true><<<dim3(blocks), dim3(kVadThreads), 0, stream>>>(x, len, row0, n, dc, out);
+    else
+      sfe_vad_frames_kernel<S, false><<<dim3(blocks), dim3(kVadThreads), 0, stream>>>(x, len, row0, n, dc, out);
+    return hipGetLastError();
+  });
 }
 
 }  // namespace
@@ -97,10 +101,9 @@ hipError_t launch_vad_frames(const void* samples, int pcm, float pcm_scale, int6
   const int64_t n = vad_num_windows(len);
   if (n == 0) return hipSuccess;
   const Decode dc{pcm_scale, 1.0f / pcm_scale, 1.0 / (double)pcm_scale};
-  if (pcm == kPcmI16) launch_vad<int16_t>(samples, len, n, dc, out, stream);
-  else if (pcm == kPcmI32) launch_vad<int32_t>(samples, len, n, dc, out, stream);
-  else launch_vad<float>(samples, len, n, dc, out, stream);
-  return hipGetLastError();
+  if (pcm == kPcmI16) return launch_vad<int16_t>(samples, len, n, dc, out, stream);
+  if (pcm == kPcmI32) return launch_vad<int32_t>(samples, len, n, dc, out, stream);
+  return launch_vad<float>(samples, len, n, dc, out, stream);
 }
 
 }  // namespace sfe

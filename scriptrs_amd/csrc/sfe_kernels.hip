@@ -973,13 +973,13 @@ __device__ __forceinline__ void norm_finish(const float* __restrict__ raw, const
 }
 
 // Workgroups [0, 8 n_segs): the long items' segments; the rest normalise the
-// other items.
+// other items.  A launch runs those from `first` on.
 template <bool SHIFT, int N, typename O>
 __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_long_kernel(
-    const float* __restrict__ raw, const Item* __restrict__ items, int n_segs, const int32_t* __restrict__ seg_item,
-    double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
+    const float* __restrict__ raw, const Item* __restrict__ items, int first, int n_segs,
+    const int32_t* __restrict__ seg_item, double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
   __shared__ NormLds<kNormMainWaves> lds;
-  const int b = blockIdx.x, rest = b - kSlabs * n_segs;
+  const int b = first + blockIdx.x, rest = b - kSlabs * n_segs;
   if (rest < 0)
     with_shift<SHIFT>(items[seg_item[b / kSlabs]],
                       [&](auto s) { norm_segment<s()>(raw, items, seg_item, b, parts, lds); });
@@ -990,10 +990,10 @@ __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_long_kernel(
 
 template <bool SHIFT, typename O>
 __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_finish_kernel(
-    const float* __restrict__ raw, const Item* __restrict__ items, const int32_t* __restrict__ seg_item,
+    const float* __restrict__ raw, const Item* __restrict__ items, int first, const int32_t* __restrict__ seg_item,
     const double2* __restrict__ parts, int pad_to, O* __restrict__ out) {
   __shared__ NormLds<kNormMainWaves> lds;
-  const int b = blockIdx.x;
+  const int b = first + blockIdx.x;
   with_shift<SHIFT>(items[seg_item[b / kSlabs]],
                     [&](auto s) { norm_finish<s()>(raw, items, seg_item, b, parts, pad_to, out, lds); });
 }
@@ -1128,40 +1128,47 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
                          hipStream_t stream) {
   using S = NormShape<kNormMainWaves>;
   using SW = NormShape<kNormWideWaves>;
-  const unsigned blocks = (unsigned)((int64_t)n_items * kSlabs);
+  const int64_t blocks = (int64_t)n_items * kSlabs, seg_blocks = (int64_t)n_segs * kSlabs;
+  if (blocks + seg_blocks > INT32_MAX) return hipErrorInvalidValue;  // (the kernels' 32-bit workgroup numbers)
   if (n_segs > 0) {
     // Long items among them: their segments' sums beside the other items,
     // then the segments themselves.
-    const unsigned seg_blocks = (unsigned)((int64_t)n_segs * kSlabs);
-    sfe_norm_long_kernel<SHIFT, kNormRegFrames / S::kSpan, O>
-        <<<dim3(seg_blocks + blocks), dim3(S::kThreads), 0, stream>>>(raw, items, n_segs, seg_item, parts, pad_to,
-                                                                      out);
-    hipError_t e = hipGetLastError();
+    const hipError_t e = for_launches(seg_blocks + blocks, S::kThreads, [&](int64_t first, unsigned n) {
+      sfe_norm_long_kernel<SHIFT, kNormRegFrames / S::kSpan, O><<<dim3(n), dim3(S::kThreads), 0, stream>>>(
+          raw, items, (int)first, n_segs, seg_item, parts, pad_to, out);
+      return hipGetLastError();
+    });
     if (e != hipSuccess) return e;
-    sfe_norm_finish_kernel<SHIFT, O><<<dim3(seg_blocks), dim3(S::kThreads), 0, stream>>>(raw, items, seg_item, parts,
-                                                                                        pad_to, out);
-    return hipGetLastError();
+    return for_launches(seg_blocks, S::kThreads, [&](int64_t first, unsigned n) {
+      sfe_norm_finish_kernel<SHIFT, O><<<dim3(n), dim3(S::kThreads), 0, stream>>>(raw, items, (int)first, seg_item,
+                                                                                 parts, pad_to, out);
+      return hipGetLastError();
+    });
   }
   // (SHIFT has no 4-wave kernels: tasks that share frames are mostly of one
   // length, where the 8-wave form is the faster one, and it loses 4% at most)
   if (SHIFT || norm_wide(n_items, max_T, sum_T, cus)) {
-    const dim3 grid(blocks), block(SW::kThreads);
-    if (max_T <= SW::kSpan * 8)
-      sfe_norm_wide_kernel<SHIFT, 8, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
-    else if (max_T <= SW::kSpan * 12)
-      sfe_norm_wide_kernel<SHIFT, 12, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
-    else
-      sfe_norm_wide_kernel<SHIFT, 16, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
-    return hipGetLastError();
+    return for_launches(blocks, SW::kThreads, [&](int64_t first, unsigned n) {
+      const Item* it = items + first / kSlabs;
+      const dim3 grid(n), block(SW::kThreads);
+      if (max_T <= SW::kSpan * 8) sfe_norm_wide_kernel<SHIFT, 8, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+      else if (max_T <= SW::kSpan * 12)
+        sfe_norm_wide_kernel<SHIFT, 12, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+      else sfe_norm_wide_kernel<SHIFT, 16, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+      return hipGetLastError();
+    });
   }
-  const dim3 grid(blocks), block(S::kThreads);
   // Registers per lane sized to the longest item (N float4s hold kSpan N
   // frames).
-  if (max_T <= S::kSpan * 8) sfe_norm_kernel<8, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
-  else if (max_T <= S::kSpan * 16) sfe_norm_kernel<16, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
-  else if (max_T <= S::kSpan * 24) sfe_norm_kernel<24, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
-  else sfe_norm_kernel<32, O><<<grid, block, 0, stream>>>(raw, items, pad_to, out);
-  return hipGetLastError();
+  return for_launches(blocks, S::kThreads, [&](int64_t first, unsigned n) {
+    const Item* it = items + first / kSlabs;
+    const dim3 grid(n), block(S::kThreads);
+    if (max_T <= S::kSpan * 8) sfe_norm_kernel<8, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+    else if (max_T <= S::kSpan * 16) sfe_norm_kernel<16, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+    else if (max_T <= S::kSpan * 24) sfe_norm_kernel<24, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+    else sfe_norm_kernel<32, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+    return hipGetLastError();
+  });
 }
 
 hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, bool shifted,

@@ -163,28 +163,29 @@ struct PinBuf {
 };
 
 // Pinned staging of the calls' tables, read by their uploads: a buffer of two
-// halves.  take() hands out consecutive pieces of the current half; when it is
-// full, an event on the caller's stream marks the end of its uploads, and the
-// other half is free once its own event (a half ago) has passed.  An event
-// after every upload, waited for by the next call, cost each call a marker
-// between its upload and its first kernel (5.6 us on the device) and held the
-// host to one call ahead.  The calls of a context are ordered after each
-// other, also across streams, so the event covers the whole half.  A piece
-// larger than a half takes the whole buffer, waiting for it on both sides.
+// halves, each with room for the largest piece.  take() hands out consecutive
+// pieces of the current half; when it is full, an event on the caller's stream
+// marks the end of its uploads, and the other half is free once its own event
+// (a half ago) has passed.  So the host waits at most for the call before the
+// previous one.  An event after every upload, waited for by the next call, cost
+// each call a marker between its upload and its first kernel (5.6 us on the
+// device) and held the host to one call ahead.  The calls of a context are
+// ordered after each other, also across streams, so the event covers the whole
+// half.
 struct PinRing {
   char* ptr = nullptr;
   size_t half = 0, at = 0;  // at: bytes used of the current half
   int cur = 0;
-  bool whole = false;         // the last piece spans both halves
   hipEvent_t ev[2] = {nullptr, nullptr};
   bool pending[2] = {false, false};
+  static size_t rounded(size_t bytes) { return (std::max(bytes, (size_t)2048) + 255) / 256 * 256; }
   hipError_t wait(int h) {
     if (!pending[h]) return hipSuccess;
     pending[h] = false;
     return hipEventSynchronize(ev[h]);
   }
-  // A buffer of at least `bytes`.  Growing waits for the device: uploads from
-  // the old one may be queued on any stream.
+  // Room for pieces of up to `bytes`.  Growing waits for the device: uploads
+  // from the old buffer may be queued on any stream.
   hipError_t reserve(size_t bytes) {
     hipError_t e;
     for (int h = 0; h < 2; ++h)
@@ -192,7 +193,7 @@ struct PinRing {
         ev[h] = nullptr;
         return e;
       }
-    const size_t want = (std::max(bytes, (size_t)4096) + 511) / 512 * 256;  // a half
+    const size_t want = rounded(bytes);
     if (want <= half) return hipSuccess;
     if (ptr) {
       if ((e = hipDeviceSynchronize()) != hipSuccess) return e;
@@ -208,7 +209,6 @@ struct PinRing {
     half = want;
     at = 0;
     cur = 0;
-    whole = false;
     pending[0] = pending[1] = false;
     return hipSuccess;
   }
@@ -217,21 +217,13 @@ struct PinRing {
   hipError_t take(size_t bytes, hipStream_t stream, char** out) {
     hipError_t e = reserve(bytes);
     if (e != hipSuccess) return e;
-    const size_t n = (bytes + 255) / 256 * 256;
+    const size_t n = rounded(bytes);
     if (at + n > half) {
       if ((e = hipEventRecord(ev[cur], stream)) != hipSuccess) return e;
       pending[cur] = true;
-      if ((whole || n > half) && (e = wait(cur)) != hipSuccess) return e;
+      if ((e = wait(cur ^ 1)) != hipSuccess) return e;
       cur ^= 1;
-      if ((e = wait(cur)) != hipSuccess) return e;
       at = 0;
-      whole = n > half;
-      if (whole) {
-        cur = 1;
-        at = half;  // full
-        *out = ptr;
-        return hipSuccess;
-      }
     }
     *out = ptr + (size_t)cur * half + at;
     at += n;
@@ -498,7 +490,6 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
   if (!same) {
     ctx->meta_items.clear();
     SFE_HIP(ctx->meta.reserve(mbytes + 16));
-    SFE_HIP(ctx->h_meta.reserve(2 * mbytes));
     char* stage = nullptr;
     SFE_HIP(ctx->h_meta.take(mbytes, stream, &stage));
     memcpy(stage, table.data(), tbytes);
@@ -939,9 +930,8 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
       SFE_HIP(sfe::noalloc_scratch(ctx->device, &na));
       ctx->noalloc = static_cast<unsigned char*>(na);
     }
-    if (2 * ctx->h_meta.half <
-            entries * sizeof(Item) + (sfe::kMaxLogmelWaves + sfe::kNoAllocMaxSegs) * sizeof(int32_t) ||
-        ctx->na_in.capacity() < (size_t)n)
+    const size_t most = entries * sizeof(Item) + (sfe::kMaxLogmelWaves + sfe::kNoAllocMaxSegs) * sizeof(int32_t);
+    if (ctx->h_meta.half < most || ctx->na_in.capacity() < (size_t)n)
       return fail(SFE_HIP_ERROR, "context has no reserved planner buffers");
     int64_t fo = 0, own_tiles = 0;
     frame_offsets[0] = 0;
@@ -957,8 +947,7 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
     SFE_HIP(order_after_last(ctx, s));
     SFE_HIP(sfe::noalloc_order(ctx->device, s));
     char* stage = nullptr;
-    SFE_HIP(ctx->h_meta.take(entries * sizeof(Item) + (sfe::kMaxLogmelWaves + sfe::kNoAllocMaxSegs) * sizeof(int32_t),
-                             s, &stage));
+    SFE_HIP(ctx->h_meta.take(most, s, &stage));
     Item* table = reinterpret_cast<Item*>(stage);
     size_t n_lm = 0;
     bool share = ctx->share;

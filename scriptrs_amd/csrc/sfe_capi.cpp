@@ -274,6 +274,7 @@ struct sfe_ctx {
   hipEvent_t ev_last = nullptr;
   bool has_last = false;
   bool last_marked = false;   // ev_last marks the end of the previous call
+  bool unsettled = false;     // a call has queued work that mark_last does not cover yet (see settle)
   bool multi_stream = false;  // calls have come on more than one stream
   hipStream_t last_stream = nullptr;  // the stream the previous call's device work ran on
   PinRing h_meta;
@@ -315,6 +316,18 @@ struct sfe_ctx {
 
 namespace {
 
+// A call that fails after it has queued work leaves that work, its table's
+// upload among it, on its stream with nothing recorded behind it.  From its
+// first queued operation to mark_last the context is unsettled, and a call that
+// finds it so waits for the device first.
+hipError_t settle(sfe_ctx* ctx) {
+  if (!ctx->unsettled) return hipSuccess;
+  const hipError_t e = hipDeviceSynchronize();
+  if (e != hipSuccess) return e;
+  ctx->unsettled = ctx->has_last = false;
+  return hipSuccess;
+}
+
 // Orders this call's work on `stream` after the context's previous call (the
 // calls share the item table and the raw scratch).  Nothing is ever enqueued
 // on an earlier call's stream, which its owner may have destroyed since.
@@ -325,7 +338,10 @@ namespace {
 //   launch-bound calls about 3 us: one 10 s clip 0.0156 -> 0.0189 ms), so the
 //   first switch waits on the host for the device to drain (work on a
 //   destroyed stream included), and from then on every call records ev_last.
+// * The previous call failed: settle.
 hipError_t order_after_last(sfe_ctx* ctx, hipStream_t stream) {
+  hipError_t e = settle(ctx);
+  if (e != hipSuccess) return e;
   if (!ctx->has_last || stream == ctx->last_stream) return hipSuccess;
   if (ctx->last_marked) return hipStreamWaitEvent(stream, ctx->ev_last, 0);
   ctx->multi_stream = true;
@@ -335,7 +351,6 @@ hipError_t order_after_last(sfe_ctx* ctx, hipStream_t stream) {
 // The call just enqueued ran on `stream`; a context that has used more than
 // one stream marks its end there with ev_last.
 hipError_t mark_last(sfe_ctx* ctx, hipStream_t stream) {
-  ctx->has_last = false;
   ctx->last_marked = false;
   if (ctx->multi_stream) {
     hipError_t e = hipEventRecord(ctx->ev_last, stream);
@@ -344,6 +359,7 @@ hipError_t mark_last(sfe_ctx* ctx, hipStream_t stream) {
   }
   ctx->has_last = true;
   ctx->last_stream = stream;
+  ctx->unsettled = false;
   return hipSuccess;
 }
 
@@ -452,6 +468,7 @@ WaveTable wave_table(const Item* lm, size_t n_lm, int cus) {
 int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, int32_t out_dtype, void* out,
               hipStream_t stream, int pad_to = 0) {
   SFE_HIP(order_after_last(ctx, stream));
+  ctx->unsettled = true;
   // one table: the log-mel entries, then the normalisation entries
   if (!(ctx->plan_share == ctx->share && ctx->plan_in.size() == items.size() &&
         memcmp(ctx->plan_in.data(), items.data(), items.size() * sizeof(Item)) == 0)) {
@@ -747,6 +764,10 @@ int sfe_extract(sfe_ctx* ctx, const float* audio, int64_t len, float* out, int64
     const int64_t nout = T * sfe::kMel;
     if (out_capacity < nout) return fail(SFE_INVALID_ARG, "output buffer too small");
     const size_t in_bytes = (size_t)len * sizeof(float), out_bytes = (size_t)nout * sizeof(float);
+    std::vector<Item> items;
+    int64_t start = 0, tiles = 0, fo[2];
+    if ((rc = build_items(&start, &len, 1, &items, fo, &tiles))) return rc;
+    SFE_HIP(settle(ctx));  // (the copy of a failed call may still read the staging)
     SFE_HIP(ctx->io_in.reserve(in_bytes));
     SFE_HIP(ctx->io_out.reserve(out_bytes));
     SFE_HIP(ctx->h_io_in.reserve(in_bytes));
@@ -755,9 +776,6 @@ int sfe_extract(sfe_ctx* ctx, const float* audio, int64_t len, float* out, int64
     hipStream_t s = ctx->s_compute;
     parallel_memcpy(ctx->h_io_in.ptr, audio, in_bytes);
     SFE_HIP(hipMemcpyAsync(ctx->io_in.ptr, ctx->h_io_in.ptr, in_bytes, hipMemcpyHostToDevice, s));
-    std::vector<Item> items;
-    int64_t start = 0, tiles = 0, fo[2];
-    if ((rc = build_items(&start, &len, 1, &items, fo, &tiles))) return rc;
     if ((rc = run_items(ctx, f32_source(static_cast<float*>(ctx->io_in.ptr)), items, SFE_F32, ctx->io_out.ptr, s)))
       return rc;
     SFE_HIP(hipMemcpyAsync(ctx->h_io_out.ptr, ctx->io_out.ptr, out_bytes, hipMemcpyDeviceToHost, s));
@@ -946,6 +964,7 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
     }
     SFE_HIP(order_after_last(ctx, s));
     SFE_HIP(sfe::noalloc_order(ctx->device, s));
+    ctx->unsettled = true;
     char* stage = nullptr;
     SFE_HIP(ctx->h_meta.take(most, s, &stage));
     Item* table = reinterpret_cast<Item*>(stage);
@@ -976,9 +995,10 @@ int sfe_extract_chunks_noalloc(sfe_ctx* ctx, const float* recording, int64_t len
     SFE_HIP(sfe::launch_upload(table, d_table, sbytes + (size_t)n_segs * sizeof(int32_t), s));
     rc = launch_pair(ctx, f32_source(recording), table, d_table, (int)n_lm, table + n_lm, d_table + n_lm, n, segs, raw, out,
                      out_dtype, 0, s, kBoth, false, d_wave);
+    // (a failed launch leaves the upload queued: other contexts wait for it too)
+    SFE_HIP(sfe::noalloc_mark(ctx->device, s));
     if (rc) return rc;
     SFE_HIP(mark_last(ctx, s));
-    SFE_HIP(sfe::noalloc_mark(ctx->device, s));
     return SFE_OK;
   });
 }
@@ -1005,6 +1025,7 @@ int sfe_vad_frames(sfe_ctx* ctx, const void* recording, int32_t pcm_format, int3
     std::lock_guard<std::mutex> lock(ctx->mu);
     hipStream_t s = static_cast<hipStream_t>(stream);
     SFE_HIP(order_after_last(ctx, s));
+    ctx->unsettled = true;
     SFE_HIP(sfe::launch_vad_frames(src.ptr, src.pcm, src.scale, len, out, s));
     SFE_HIP(mark_last(ctx, s));
     return SFE_OK;
@@ -1113,6 +1134,7 @@ int sfe_extract_chunks_streamed_pcm(sfe_ctx* ctx, const void* host_recording, in
     hipStream_t sc = ctx->s_compute, sx = ctx->s_copy;
     SFE_HIP(order_after_last(ctx, sc));
     SFE_HIP(order_after_last(ctx, sx));
+    ctx->unsettled = true;
     char* ring = static_cast<char*>(ctx->win.ptr);
     // Batch bi's samples into half (bi & 1) of the ring, on the copy stream.
     auto issue_copy = [&](size_t bi) -> int {
@@ -1249,7 +1271,7 @@ int sfe_extract_chunks_streamed_pcm(sfe_ctx* ctx, const void* host_recording, in
     }
     SFE_HIP(hipStreamSynchronize(sc));
     SFE_HIP(hipStreamSynchronize(sx));
-    ctx->has_last = false;  // everything has completed
+    ctx->has_last = ctx->unsettled = false;  // everything has completed
     return SFE_OK;
   });
 }

@@ -17,6 +17,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <functional>
 #include <memory>
 #include <string>
@@ -299,6 +300,70 @@ int main(int argc, char** argv) {
         }
         check_all("ahead");
       }
+  } else if (name == "failed") {
+    // a call whose normalisation does not launch leaves its upload and its
+    // log-mel queued on its stream; the calls after it come on another one
+    auto fails = [&](Call* c, hipStream_t s, bool noalloc = false) {
+      g_fail_norm = 1;
+      expect(run(c, s, noalloc) == SFE_HIP_ERROR, "the launch did not fail");
+      g_fail_norm = 0;
+      std::fill(c->out.begin(), c->out.end(), -1.0f);
+    };
+    // the first call of the context fails; then one that failed after others.
+    // The same table again: its upload must have run.
+    for (int k = 0; k < 3; ++k) {
+      Call* c = make(20 + k, 1600, k);
+      fails(c, a);
+      expect(run(c, b) == SFE_OK, "call failed");
+      hipStreamSynchronize(b);
+      check(c, "same table after a failed call");
+      check_all("same table after a failed call");
+    }
+    // other tables: the failed call's upload must not come after theirs
+    for (int k = 0; k < 3; ++k) {
+      fails(make(20, 1600, 40 + k), a);
+      g_calls.pop_back();
+      Call* c = make(30, 1600, k);
+      expect(run(c, b) == SFE_OK, "call failed");
+      hipStreamSynchronize(b);
+      drain();
+      std::fill(c->out.begin(), c->out.end(), -1.0f);
+      expect(run(c, b) == SFE_OK, "call failed");
+      check_all("other table after a failed call");
+    }
+    // a clip from host memory, a streamed recording
+    std::vector<float> x(1600), y(128 * 11);
+    g_fail_norm = 1;
+    expect(sfe_extract(g_ctx, x.data(), 1600, y.data(), (int64_t)y.size()) == SFE_HIP_ERROR, "the launch did not fail");
+    g_waits = 0;
+    expect(sfe_extract(g_ctx, x.data(), 1600, y.data(), (int64_t)y.size()) == SFE_OK, "call failed");
+    expect(g_waits == 2, "a clip after a failed one waits for it before it writes the staging");
+    g_fail_norm = 1;
+    std::vector<float> host;
+    expect(run_streamed(make(40, 1600, 3), &host) == SFE_HIP_ERROR, "the launch did not fail");
+    g_calls.pop_back();
+    Call* c = make(30, 1600, 5);
+    expect(run(c, b) == SFE_OK, "call failed");
+    hipStreamSynchronize(b);
+    drain();
+    std::fill(c->out.begin(), c->out.end(), -1.0f);
+    expect(run(c, b) == SFE_OK, "call failed");
+    check_all("after a failed streamed call");
+    // the static scratch, from another context: its upload, then the failed
+    // call's as late as it may come, then its kernels
+    sfe_ctx* other = g_ctx;
+    fails(make(25, 1600, 7), a, true);
+    g_calls.pop_back();
+    if (sfe_create(&cfg, 0, &g_ctx)) return 2;
+    expect(run(make(25, 1600, 8), b, true) == SFE_OK, "call failed");
+    run_to(::st(b), ::st(b)->ops.size() - 2);
+    check_all("static scratch after a failed call");
+    sfe_destroy(other);
+    // and a context without failures waits for nothing
+    g_waits = 0;
+    for (int k = 0; k < 4; ++k) run(make(5, 1600, 20 + k), b);
+    expect(g_waits == 0, "calls without a failure wait");
+    check_all("after");
   } else {
     return 3;
   }

@@ -477,14 +477,16 @@ int run_items(sfe_ctx* ctx, const Source& src, const std::vector<Item>& items, i
     ws.reserve(items.size());
     std::vector<Item> table((size_t)(sfe::kPlanEntriesPerItem + 1) * items.size());
     size_t n_lm = 0;
-    ctx->plan_tiles = sfe::plan_table(items.data(), n, ctx->share, &ws, table.data(), &n_lm);
+    const int64_t tiles = sfe::plan_table(items.data(), n, ctx->share, &ws, table.data(), &n_lm);
     sfe::order_norm(table.data() + n_lm, n);
     table.resize(n_lm + items.size());
-    ctx->plan_segs = sfe::norm_segments(table.data() + n_lm, n, nullptr);
-    if (ctx->plan_segs > INT32_MAX / 8) return fail(SFE_INVALID_ARG, "batch too large for one launch");
-    ctx->plan_n_lm = n_lm;
+    const int64_t plan_segs = sfe::norm_segments(table.data() + n_lm, n, nullptr);
+    if (plan_segs > INT32_MAX / 8) return fail(SFE_INVALID_ARG, "batch too large for one launch");
+    ctx->plan_in = items;  // (may throw: before anything of the old plan changes)
     ctx->plan_table.swap(table);
-    ctx->plan_in = items;
+    ctx->plan_n_lm = n_lm;
+    ctx->plan_tiles = tiles;
+    ctx->plan_segs = plan_segs;
     ctx->plan_share = ctx->share;
   }
   const std::vector<Item>& table = ctx->plan_table;

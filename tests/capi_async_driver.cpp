@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <functional>
 #include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -47,6 +48,13 @@ static long g_kernels_run = 0;  // by host waits
 static long g_waits = 0;        // host waits that found something to run
 static bool g_capturing = false;
 static int g_fail_norm = 0;     // the next launches of the normalisation that fail
+static long g_fail_new = -1;    // the allocation that fails (counted down to 0)
+void* operator new(size_t n) {
+  if (g_fail_new >= 0 && g_fail_new-- == 0) throw std::bad_alloc();
+  return malloc(n);
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 static ihipStream_t* st(hipStream_t s) { return s ? s : &g_null; }
 static void run_to(ihipStream_t* s, size_t n) {
@@ -364,6 +372,26 @@ int main(int argc, char** argv) {
     for (int k = 0; k < 4; ++k) run(make(5, 1600, 20 + k), b);
     expect(g_waits == 0, "calls without a failure wait");
     check_all("after");
+  } else if (name == "memory") {
+    // each of a call's host allocations fails in turn: the calls after it, with
+    // the plan from before it and with its own, are right
+    warm(300, 1600);
+    int failures = 0;
+    for (int k = 0; k < 100; ++k) {
+      Call* before = make(60, 1600, 3 * k);
+      expect(run(before, a) == SFE_OK, "call failed");
+      Call* c = make(400 + 10 * k, 1603, 3 * k + 1);  // (more tasks than any before: every list grows)
+      g_fail_new = k;
+      const int rc = run(c, a);
+      g_fail_new = -1;
+      drain();
+      std::fill(before->out.begin(), before->out.end(), -1.0f);
+      expect(run(before, a) == SFE_OK && run(c, a) == SFE_OK, "call failed");
+      check_all("after a failed allocation");
+      if (rc == SFE_OK) break;
+      ++failures;
+    }
+    expect(failures > 5 && failures < 100, "allocations failed");
   } else {
     return 3;
   }

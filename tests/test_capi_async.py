@@ -25,7 +25,7 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["turns", "streams", "grow", "mixed", "ahead", "failed"])
+@pytest.mark.parametrize("scenario", ["turns", "streams", "grow", "mixed", "ahead", "failed", "memory"])
 def test_queued_calls(driver, scenario):
     r = subprocess.run([driver, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip().endswith("bad 0"), r.stdout[-3000:] + r.stderr[-3000:]

@@ -290,6 +290,36 @@ void logmel_wave_items(const Item* items, int n_items, int unit0, int n_units, L
 hipError_t launch_logmel(const void* samples, int pcm, float pcm_scale, const Item* items, int n_items, int unit0,
                          int n_units, const DevTables* tables, int schedule, float preemph, float* raw_out, int cus,
                          const int32_t* wave_item, hipStream_t stream);
+// Workgroup form of a normalisation launch without long items: 8 waves (128
+// frames per round, 33 KB of LDS for the 512-frame transpose chunks, half the
+// registers per lane, 3 per CU) or 4 (64 frames per round, 4 per CU).  With 8,
+// each item is loaded, reduced and stored by twice the waves, but fewer items
+// are resident at once, and items of few rounds leave waves without a quad.
+// Normalisation times, 4-wave / 8-wave (of items up to 512 frames between
+// events, which add about 2 us):
+// * past 512 frames: one 10 s clip 6.8 / 5.3 us, 40 ragged clips 12.2 / 10.2,
+//   10 min long form (47 chunks) 18.0 / 15.2, 64 x 15 s 20.3 / 18.5, 1 h (280
+//   chunks) 77 / 72, 8 h to bf16 436 / 428; but 128 clips of 1-15 s 18.9 / 20.5,
+//   256 of 1-20 s 50.2 / 52, 128 of 7.5-15 s 25.0 / 26.1: once the items no
+//   longer fit at 3 per CU, the 8-wave form needs them of nearly one length
+//   (measured down to 7/8 of the longest on average: 128 of 11-15 s 30.6 /
+//   30.1);
+// * up to 256 frames: 1 clip of 2 s 6.8 / 7.3, 48 of 2 s 8.2 / 9.1, 97 of 1 s
+//   9.0 / 11.3, 300 of 0.5 s 16.3 / 20.9, 1,200 of 2 s 55 / 64;
+// * between, 8 waves only while every workgroup has a CU to itself (32 x 4 s
+//   8.5 / 8.2, 48 x 4 s 9.5 / 9.9, 96 x 5 s 12.6 / 13.0, 128 x 5 s 14.1 / 14.4) or
+//   where 4-wave ones of nearly 512 frames no longer fit at 4 per CU (160 x 5 s
+//   18.6 / 17.9, 1,200 x 5 s 108 / 103; 600 x 4 s 44.3 / 45.9).
+constexpr int kNormShortFrames = 512;
+constexpr int kNormWidePerCu = 3;
+inline bool norm_wide(int n_items, int max_T, int64_t sum_T, int cus) {
+  const int64_t groups = (int64_t)n_items * (kMel / 16);  // one per slab of 16 features
+  const bool even = 8 * sum_T >= (int64_t)7 * max_T * n_items;
+  if (groups <= cus) return max_T > kNormShortFrames / 2;
+  if (max_T <= kNormShortFrames) return even && 8 * max_T > 7 * kNormShortFrames && groups > (int64_t)4 * cus;
+  return groups <= (int64_t)kNormWidePerCu * cus || even;
+}
+
 // Normalises raw (f32 log2 values in 16-frame tiles, see Item) per (item, feature)
 // and writes feature-major [128][T] per item to out (f32, must not alias
 // raw) or bf16 (uint16_t*) when out_bf16 is set.  max_T: the longest item's

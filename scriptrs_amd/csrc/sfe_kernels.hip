@@ -841,14 +841,7 @@ __global__ __launch_bounds__(kUploadThreads) void sfe_upload_kernel(const uint4*
 // Workgroups of kNormMainWaves waves; workgroup b normalises slab b % 8 of
 // item b / 8.
 constexpr int kNormMainWaves = 4;
-
-template <int N, typename O>
-__global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_kernel(const float* __restrict__ raw,
-                                                                       const Item* __restrict__ items, int pad_to,
-                                                                       O* __restrict__ out) {
-  __shared__ NormLds<kNormMainWaves> lds;
-  norm_body<0, kNormMainWaves, N>(raw, items, blockIdx.x, pad_to, out, lds);
-}
+constexpr int kNormWideWaves = 8;
 
 // Runs body<shift> for the item's own shift: one instance a value, each with
 // its loads and nothing to choose per load.  (Chosen inside one instance, the
@@ -865,6 +858,16 @@ __device__ __forceinline__ void with_shift(const Item& it, F&& body) {
   else if (s == 1) body(std::integral_constant<int, 1>());
   else if (s == 2) body(std::integral_constant<int, 2>());
   else body(std::integral_constant<int, 3>());
+}
+
+template <bool SHIFT, int N, typename O>
+__global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_kernel(const float* __restrict__ raw,
+                                                                       const Item* __restrict__ items, int pad_to,
+                                                                       O* __restrict__ out) {
+  __shared__ NormLds<kNormMainWaves> lds;
+  const int b = blockIdx.x;
+  with_shift<SHIFT>(items[b / kSlabs],
+                    [&](auto s) { norm_body<s(), kNormMainWaves, N>(raw, items, b, pad_to, out, lds); });
 }
 
 // Long items, in segments of seg_frames(T) frames, chunks of 512 in registers.
@@ -998,23 +1001,6 @@ __global__ __launch_bounds__(64 * kNormMainWaves) void sfe_norm_finish_kernel(
                     [&](auto s) { norm_finish<s()>(raw, items, seg_item, b, parts, pad_to, out, lds); });
 }
 
-// 8-wave workgroups (128 frames per round, 33 KB of LDS for the 512-frame
-// transpose chunks, half the registers per lane, 3 per CU) against 4-wave
-// ones (4 per CU in the 24-round class): each item is loaded, reduced and
-// stored by twice the waves, but fewer items are resident at once.
-// Normalisation times, 4-wave / 8-wave: one clip 6.8 / 5.3 us, 40 ragged clips
-// 12.2 / 10.2, 10 min long form (47 chunks) 18.0 / 15.2, 64 x 15 s 20.3 /
-// 18.5, 1 h (280 chunks) 77 / 72, 8 h to bf16 436 / 428; but 128 clips of
-// 1-15 s 18.9 / 20.5, 256 of 1-20 s 50.2 / 52, 128 of 7.5-15 s 25.0 / 26.1:
-// once the items no longer fit at 3 per CU, the 8-wave form needs them of
-// nearly one length (measured down to 7/8 of the longest on average: 128 of
-// 11-15 s 30.6 / 30.1).
-constexpr int kNormWideWaves = 8;
-constexpr int kNormWidePerCu = 3;
-inline bool norm_wide(int n_items, int max_T, int64_t sum_T, int cus) {
-  return (int64_t)n_items * kSlabs <= (int64_t)kNormWidePerCu * cus || 8 * sum_T >= (int64_t)7 * max_T * n_items;
-}
-
 template <bool SHIFT, int N, typename O>
 __global__ __launch_bounds__(64 * kNormWideWaves) void sfe_norm_wide_kernel(const float* __restrict__ raw,
                                                                             const Item* __restrict__ items,
@@ -1128,6 +1114,7 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
                          hipStream_t stream) {
   using S = NormShape<kNormMainWaves>;
   using SW = NormShape<kNormWideWaves>;
+  static_assert(kNormShortFrames == S::kSpan * 8, "the 4-wave form's smallest class");
   const int64_t blocks = (int64_t)n_items * kSlabs, seg_blocks = (int64_t)n_segs * kSlabs;
   if (blocks + seg_blocks > INT32_MAX) return hipErrorInvalidValue;  // (the kernels' 32-bit workgroup numbers)
   if (n_segs > 0) {
@@ -1145,9 +1132,10 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
       return hipGetLastError();
     });
   }
-  // (SHIFT has no 4-wave kernels: tasks that share frames are mostly of one
-  // length, where the 8-wave form is the faster one, and it loses 4% at most)
-  if (SHIFT || norm_wide(n_items, max_T, sum_T, cus)) {
+  // (SHIFT has 4-wave kernels for short items only: 1,172 windows of 2 s every
+  // 0.51 s 49 us, 66 with 8 waves.  Longer tasks that share frames are mostly of
+  // one length, where the 8-wave form is the faster one, and it loses 4% at most.)
+  if ((SHIFT && max_T > kNormShortFrames) || norm_wide(n_items, max_T, sum_T, cus)) {
     return for_launches(blocks, SW::kThreads, [&](int64_t first, unsigned n) {
       const Item* it = items + first / kSlabs;
       const dim3 grid(n), block(SW::kThreads);
@@ -1163,10 +1151,13 @@ hipError_t launch_norm_t(const float* raw, const Item* items, int n_items, int m
   return for_launches(blocks, S::kThreads, [&](int64_t first, unsigned n) {
     const Item* it = items + first / kSlabs;
     const dim3 grid(n), block(S::kThreads);
-    if (max_T <= S::kSpan * 8) sfe_norm_kernel<8, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
-    else if (max_T <= S::kSpan * 16) sfe_norm_kernel<16, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
-    else if (max_T <= S::kSpan * 24) sfe_norm_kernel<24, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
-    else sfe_norm_kernel<32, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+    if (SHIFT || max_T <= S::kSpan * 8) {
+      sfe_norm_kernel<SHIFT, 8, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+    } else if constexpr (!SHIFT) {
+      if (max_T <= S::kSpan * 16) sfe_norm_kernel<false, 16, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+      else if (max_T <= S::kSpan * 24) sfe_norm_kernel<false, 24, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+      else sfe_norm_kernel<false, 32, O><<<grid, block, 0, stream>>>(raw, it, pad_to, out);
+    }
     return hipGetLastError();
   });
 }

@@ -1,7 +1,8 @@
 // Host run of sfe::for_launches (scriptrs_amd/csrc/sfe_internal.hpp): for
 // workgroup sizes and counts around the most that a launch holds, every
 // workgroup is in exactly one launch, in order, no launch holds 2^32 threads or
-// more, and all but the last start at a multiple of 8.  Prints "bad N".
+// more, and all but the last start at a multiple of 8.  And the rule that picks
+// the workgroup form of the normalisation, sfe::norm_wide.  Prints "bad N".
 #include <stdio.h>
 
 #include "sfe_internal.hpp"
@@ -25,6 +26,14 @@ int main() {
         bad += sfe::for_launches(blocks, threads, [&](int64_t, unsigned) { return hipErrorUnknown; }) != hipErrorUnknown;
     }
   }
+  // the workgroup form of the normalisation (sfe::norm_wide), 256 CUs: clips of
+  // one length, then ragged ones
+  struct { int n, T, wide; } forms[] = {{1, 10, 0}, {1, 256, 0}, {1, 257, 1}, {1, 2000, 1}, {32, 201, 0}, {32, 401, 1},
+                                        {33, 401, 0}, {96, 501, 0}, {128, 501, 0}, {129, 501, 1}, {300, 51, 0},
+                                        {300, 201, 0}, {2400, 201, 0}, {300, 401, 0}, {300, 448, 0}, {300, 449, 1},
+                                        {40, 513, 1}, {96, 1501, 1}, {300, 1501, 1}, {300, 2048, 1}};
+  for (auto& f : forms) bad += sfe::norm_wide(f.n, f.T, (int64_t)f.n * f.T, 256) != (f.wide != 0);
+  for (auto& f : forms) bad += sfe::norm_wide(f.n, f.T, (int64_t)f.n * f.T / 2, 256) != (f.wide && 8 * f.n <= 768);
   printf("bad %ld\n", bad);
   return bad != 0;
 }

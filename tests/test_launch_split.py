@@ -1,7 +1,9 @@
 """Calls of more workgroups than one launch holds (2^32 threads): the split
 into launches on the host (tests/launch_split_driver.cpp), and on the GPU
 batches of more clips than one normalisation launch takes in its 8-wave and
-4-wave forms, which such a launch left unwritten without an error."""
+4-wave forms, which such a launch left unwritten without an error.  The driver also pins the
+rule that picks the form.  Short clips of one length take the 4-wave form, which
+is up to a quarter faster there (300 clips of 0.5 s 16 against 21 us)."""
 import os
 import subprocess
 

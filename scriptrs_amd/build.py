@@ -11,6 +11,7 @@ import re
 import subprocess
 import sys
 import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -127,18 +128,22 @@ def build(verbose: bool = False, timestamps: bool = False) -> str:
     obj_dir = os.path.join(OBJ, "ts") if timestamps else OBJ
     lib = LIB_TS if timestamps else LIB
     os.makedirs(obj_dir, exist_ok=True)
-    objs = []
-    for src, extra in SOURCES:
-        obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
-        if timestamps and src == "sfe_kernels.hip":
-            extra = [*extra, "-DSFE_TIMESTAMPS"]
-        cmd = [HIPCC, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        subprocess.run(cmd, check=True)
-        objs.append(obj)
-        if src in MFMA_CHECKED:
-            check_asm(src, extra, verbose)
+    objs, jobs = [], []
+    # (the kernels' object and their assembly take most of the time: side by side)
+    with ThreadPoolExecutor(max_workers=4) as pool:
+        for src, extra in SOURCES:
+            obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
+            if timestamps and src == "sfe_kernels.hip":
+                extra = [*extra, "-DSFE_TIMESTAMPS"]
+            cmd = [HIPCC, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            jobs.append(pool.submit(subprocess.run, cmd, check=True))
+            objs.append(obj)
+            if src in MFMA_CHECKED:
+                jobs.append(pool.submit(check_asm, src, extra, verbose))
+    for job in jobs:
+        job.result()
     tmp = lib + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     if verbose:

@@ -185,15 +185,6 @@ struct DevTables {
   // component s % 4; each filter's first bin.
   float4 mel_w[kMelVecMax][64];
   int32_t mel_k0[kMelSlots][64];
-  // The same transform as a 16 x 16 complex FFT with an even/odd split
-  // (sfe_fft.hpp dft16_windowed, split_power), which the host check of the
-  // 16-point pieces runs: tan256[l * 16 + k1], cos256[k1 * 16 + l] of
-  // e^{-2 pi i l k1 / 256} (at cos = 0, l k1 = 64: 2^-100 and 2^100), and
-  // split twiddles e^{-2 pi i k / 512}, k < 128, as (cos, tan) for k < 64 and
-  // (sin, cos / sin) above.
-  float tan256[256];
-  float cos256[256];
-  float2 split[128];
   int32_t schedule;         // index into kMelSteps
 };
 
@@ -326,8 +317,9 @@ inline bool norm_wide(int n_items, int max_T, int64_t sum_T, int cus) {
 // frame count (sizes the kernel's register budget); sum_T: all items' frames;
 // shifted: whether any item has gshift % kQuad != 0; cus: the device's
 // compute units.  pad_to > 0: rows of pad_to frames, zero past T (the encoder
-// input layout).  n_segs, seg_item, parts: the long items' segments (norm_segments over items), the device copy
-// of their entry indexes and n_segs * kSegPartBytes of scratch.
+// input layout).  n_segs, seg_item, parts: the long items' segments
+// (norm_segments over items), the device copy of their entry indexes and
+// n_segs * kSegPartBytes of scratch.
 hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, bool shifted,
                        int cus, int pad_to, void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
                        hipStream_t stream);

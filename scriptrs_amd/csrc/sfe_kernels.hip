@@ -25,9 +25,9 @@
 //
 // What bounds it: vector issue.  An f32 MFMA takes the vector ALU with it on
 // this GPU (measured with one wave of each per SIMD: 16x16x4 32 cycles, 4x4x1
-// about 9, none of it overlapped; bf16 MFMAs do overlap), so f32 matrix
-// products pay only where they need under a third of the vector operations:
-// the 8 of the special columns here (9 cycles each, against 32 fmas), while
+// about 9, none of it overlapped; bf16 MFMAs do overlap), so 4x4x1 products
+// pay only where they are fewer than 4/9 of the vector operations, which take
+// 4 cycles each: the 8 of the special columns here (against 32 fmas), while
 // the mel sums (68 fmas a quad) left them (40 MFMAs, 86 issue slots) and a
 // first stage on them (32 16x16x4) was 20% slower than this kernel.  522
 // vector instructions a quad against 582 of the 16 x 16 complex FFT with its
@@ -353,7 +353,7 @@ void sfe_logmel_kernel(const S* __restrict__ samples, const Item* __restrict__ i
     // ---- 1. preemphasised, zero-padded samples of this wave's 4 frames
     // y[0] = x[0], y[s] = x[s] - coef * x[s-1] (separately rounded, as
     // src/frontend.rs:157 computes it), zero outside [0, L).  The previous
-    // quad's MFMA reads of this buffer were issued earlier, and LDS
+    // quad's mel reads of this buffer were issued earlier, and LDS
     // operations of a wave complete in order.
     if (sp.interior) {
 #pragma clang fp contract(off)

@@ -22,8 +22,8 @@
 // covers the union of their interior frames.  (An item that starts inside a
 // quad of the shared region finds its own quads across two of them,
 // Rounds::elem_off.)  Each item keeps its own first quad (frames 0-3) and its
-// last quads (frames past the interior), in tiles of its own.  A run is shared only if that computes fewer quads than its
-// items would alone.
+// last quads (frames past the interior), in tiles of its own.  A run is shared
+// only if that computes fewer quads than its items would alone.
 #include <algorithm>
 #include <vector>
 

@@ -43,8 +43,7 @@ def test_lengths_at_segment_edges(extractor, frames):
             assert np.all(np.abs(g - want) <= 1e-4 + 1e-3 * np.abs(want) + env), f"{frames[i]} frames"
         # a clip's features do not depend on the others of its call
         alone, _ = extractor.extract_batch(dev[off[i]:off[i + 1]].contiguous(), [0, c.size])
-        if frames[i] > 2048:
-            assert np.array_equal(alone.cpu().numpy(), g.reshape(-1)), frames[i]
+        assert np.array_equal(alone.cpu().numpy(), g.reshape(-1)), frames[i]
 
 
 def test_long_items_shared_padded_and_silent(extractor):

@@ -782,10 +782,11 @@ def test_config3_shared_frames_equal_own_frames(extractor):
 
 def test_norm_class_does_not_change_results(extractor):
     """The normalisation kernel's register class follows the batch's longest
-    item (16, 24 or 24 + 8 rounds of 64 frames in registers, or the
-    streaming path past 2048 frames); every class sums the same rounds in the
-    same groups, so 17 clips give bitwise the same features whichever longer
-    clip joins their batch (17 clips: past the 8-wave few-item variant)."""
+    item; 17 or 18 clips take the 8-wave form (8, 12 or 16 rounds of 128 frames
+    in registers) and, next to an item past 2048 frames, the 4-wave one of
+    calls with segments.  Every class sums the same quads in the same order, so
+    17 clips give bitwise the same features whichever longer clip joins their
+    batch.  (The 4-wave form's own classes: tests/test_gpu_norm_forms.py.)"""
     import torch
     rng = np.random.default_rng(77)
     lens = [int(v) for v in rng.integers(16_000, 160_000, 17)]  # at most 1000 frames
@@ -809,9 +810,9 @@ def test_norm_class_does_not_change_results(extractor):
 def test_batch_split_into_calls_is_bitwise_the_same(extractor, frames):
     """240 clips in one call (1,920 16-feature slabs of normalisation, more
     than the GPU holds workgroups at once) and the same clips in four calls
-    of 60 give bitwise the same features: each call's longest clip is in the
-    same register class (16 or 24 rounds of 64 frames), and the sums run in
-    the same groups whatever the batch.  Clips of the full batch are also
+    of 60 give bitwise the same features: the sums run in the same order
+    whatever the batch (the call of all takes the 4-wave form in its 16- or
+    24-round class, the calls of 60 the 8-wave one).  Clips of the full batch are also
     checked against the oracle."""
     import torch
     lo, hi = frames

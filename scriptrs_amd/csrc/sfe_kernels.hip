@@ -527,9 +527,18 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
 // 28, 64 clips of 480,000 samples at 48 kHz 406 / 140.
 __device__ __forceinline__ void constant_row_stats(float x0, int T, float* mean_out, float* sd_out) {
 #pragma clang fp contract(off)  // every f32 operation rounded, as the reference's
-  const float mean = __fdiv_rn(sequential_sum(x0, T), (float)T);
-  const float d = x0 - mean;
-  const float var = __fdiv_rn(sequential_sum(d * d, T), (float)T - 1.0f);
+  float a = x0, mean = 0.0f, var = 0.0f;
+#pragma unroll 1  // one copy of the sum's code: the store phase follows it
+  for (int pass = 0; pass < 2; ++pass) {
+    const float sum = sequential_sum(a, T);
+    if (pass == 0) {
+      mean = __fdiv_rn(sum, (float)T);
+      const float d = x0 - mean;
+      a = d * d;
+    } else {
+      var = __fdiv_rn(sum, (float)T - 1.0f);
+    }
+  }
   *mean_out = mean;
   *sd_out = __fsqrt_rn(var) + 1e-5f;
 }
@@ -628,7 +637,7 @@ __device__ __forceinline__ void publish_stats(double S, double Q, bool constant,
                                               float* st) {
   if (w == 0 && lane < kSlabF) {
     float mean, sd;
-    if (constant) {
+    if (__builtin_expect(constant, 0)) {
       constant_row_stats(x0, T, &mean, &sd);
     } else {
       mean = row_mean(x0, S, T);
@@ -719,6 +728,9 @@ __device__ __forceinline__ void load_rounds(const Rounds<W>& rd, float4 (&v)[N])
       __builtin_amdgcn_sched_barrier(0);  // one round's addresses at a time: they take registers beside v
     }
   }
+  // (Left to itself the scheduler moves the first uses, and their waits, up
+  // among the loads.)
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // Adds the f32 sum over a quad of (x - p) to s; elements past the item (index >= n)

@@ -1250,7 +1250,6 @@ int sfe_extract_chunks_streamed_pcm(sfe_ctx* ctx, const void* host_recording, in
     rsrc.ptr = ring;
     size_t next_norm = 0;  // group
     for (size_t bi = 0; bi < batches.size(); ++bi) {
-      const Batch& bt = batches[bi];
       const int e = (int)(bi & 1);
       if (bi > 0 && (rc = issue_copy(bi))) return rc;
       SFE_HIP(hipStreamWaitEvent(sc, ctx->ev_copied[e], 0));

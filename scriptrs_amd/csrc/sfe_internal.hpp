@@ -323,6 +323,10 @@ inline bool norm_wide(int n_items, int max_T, int64_t sum_T, int cus) {
 hipError_t launch_norm(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, bool shifted,
                        int cus, int pad_to, void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
                        hipStream_t stream);
+// launch_norm's `shifted` calls (sfe_norm_shift.hip).
+hipError_t launch_norm_shifted(const float* raw, const Item* items, int n_items, int max_T, int64_t sum_T, int cus,
+                               int pad_to, void* out, bool out_bf16, int n_segs, const int32_t* seg_item, void* parts,
+                               hipStream_t stream);
 
 // Static scratch of the allocation-free entry point (sfe_noalloc.hip): an
 // item table of up to kNoAllocMaxItems items, then kNoAllocRawBytes of raw

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import os
 import re
+import shutil
 import subprocess
 import sys
 import tempfile
@@ -20,6 +21,7 @@ OBJ = os.path.join(CSRC, "_obj")
 LIB = os.path.join(HERE, "libscriptrs_fe.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
+LD = os.path.join(os.path.dirname(os.path.realpath(shutil.which(HIPCC) or HIPCC)), "..", "lib", "llvm", "bin", "ld.lld")
 
 COMMON = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
@@ -44,12 +46,18 @@ SOURCES = [
 ]
 
 
+# The kernels of a call are one object file on the host and two code objects on
+# the GPU, of which a process loads the second with its first shifted task
+# (csrc/sfe_norm.hpp).
+JOINED = ("sfe_kernels.hip", "sfe_norm_shift.hip")
+assert tuple(src for src, _ in SOURCES[:2]) == JOINED
+
 # Kernel sources whose generated assembly is checked: for registers spilled, and
 # for MFMAs with a destination overlapping their own A or B operand.  The register allocator
 # allows that overlap (it treats the operands as read at issue); whether the
 # matrix cores read every block's operands before the destination is written
 # is not documented, so the kernels are kept free of it.
-ASM_CHECKED = ("sfe_kernels.hip", "sfe_norm_shift.hip")
+ASM_CHECKED = JOINED
 _MFMA_RE = re.compile(r"\bv_mfma\w*\s+v\[(\d+):(\d+)\],\s*v(\d+),\s*v(\d+)")
 
 
@@ -133,7 +141,7 @@ def build(verbose: bool = False, timestamps: bool = False) -> str:
     # (the kernels' object and their assembly take most of the time: side by side)
     with ThreadPoolExecutor(max_workers=4) as pool:
         for src, extra in SOURCES:
-            obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
+            obj = os.path.join(obj_dir, os.path.splitext(src)[0] + (".part.o" if src in JOINED else ".o"))
             if timestamps and src == "sfe_kernels.hip":
                 extra = [*extra, "-DSFE_TIMESTAMPS"]
             cmd = [HIPCC, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
@@ -145,6 +153,9 @@ def build(verbose: bool = False, timestamps: bool = False) -> str:
                 jobs.append(pool.submit(check_asm, src, extra, verbose))
     for job in jobs:
         job.result()
+    parts = objs[:len(JOINED)]
+    objs = [os.path.join(obj_dir, "sfe_kernels.o"), *objs[len(JOINED):]]
+    subprocess.run([LD, "-r", *parts, "-o", objs[0]], check=True)
     tmp = lib + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     if verbose:

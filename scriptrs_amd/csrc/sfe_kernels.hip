@@ -9,8 +9,8 @@
 // and writes the raw log-mel to scratch in tiles of 16 frames (8 slabs of 16
 // features, 4 consecutive frames of a feature together), in base 2 (the
 // normalisation kernel multiplies by ln 2 as it loads).
-// sfe_norm_kernel then applies normalize_columns (src/frontend.rs:225-241)
-// per (item, feature) and writes the reference's feature-major layout
+// The normalisation (sfe_norm.hpp) then applies normalize_columns
+// (src/frontend.rs:225-241) per (item, feature) and writes the reference's feature-major layout
 // ([128][T] per item).
 //
 // FFT mapping: the 512-point real FFT is 32 x 16 with tap n = 16 (b + 12) +
